@@ -11,7 +11,8 @@
  *     allocates no device memory and keeps no state between calls besides
  *     a cached per-device capability check, the fixed scratch array of
  *     tilemix_tiles_importance_noalloc, and the fixed split workspace and
- *     one ordering event per device of tilemix_attention (see there);
+ *     one ordering event per device of the attention calls (see
+ *     tilemix_attention);
  *   - `stream` is a `hipStream_t` (NULL = the default stream); all work is
  *     enqueued on it and nothing synchronises;
  *   - the return value is a `hipError_t` code (0 = hipSuccess). Argument
@@ -67,6 +68,10 @@ int tilemix_quantize_qk(const uint16_t* Q, const uint16_t* K, int8_t* Q8, int8_t
  * second kernel on `stream`. Split calls on one device are ordered through one event (each
  * waits for the previous one's merge, on any stream); a call made while
  * `stream` is being captured into a graph takes the unsplit launch.
+ * A call of M <= 16 query rows (here and in tilemix_attention_batched without
+ * a causal mask) is served by a kernel of its own, which splits the keys of
+ * its heads over workgroups of the same launch through the same workspace,
+ * ordered and unsplit under capture in the same way.
  */
 int tilemix_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* V, float* O,
                       int M, int N, int d, float score_scale, void* stream,

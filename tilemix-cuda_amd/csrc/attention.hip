@@ -1123,10 +1123,6 @@ hipError_t launch_dc(const AttnParams& p, bool vector, bool precise, hipStream_t
     return vector ? launch_vp<DC, true>(p, precise, dots, stream) : launch_vp<DC, false>(p, precise, dots, stream);
 }
 
-bool aligned(const void* pointer, std::size_t bytes) {
-    return (reinterpret_cast<std::uintptr_t>(pointer) % bytes) == 0;
-}
-
 std::size_t words_per_row(int N, int group) {
     const std::size_t key_tiles = (static_cast<std::size_t>(N) - 1) / kCellKeys + 1;
     const std::size_t groups = (key_tiles - 1) / static_cast<std::size_t>(group) + 1;
@@ -1186,16 +1182,8 @@ hipError_t launch_attention(AttnParams p, bool precise, hipStream_t stream) {
     // 32-bit buffer offsets; other shapes take the element-wise path.
     const std::int64_t k_range = (static_cast<std::int64_t>(p.N - 1) * p.k_row + p.d) * 2;
     const std::int64_t v_range = (static_cast<std::int64_t>(p.N - 1) * p.v_row + p.d) * 2;
-    bool vector = p.d % 16 == 0 && aligned(p.Q, 16) && aligned(p.K, 16) && aligned(p.V, 16) &&
-                  aligned(p.O, 16) && p.q_stride % 8 == 0 && p.k_stride % 8 == 0 &&
-                  p.v_stride % 8 == 0 && p.o_stride % 4 == 0 && p.q_row % 8 == 0 &&
-                  p.k_row % 8 == 0 && p.v_row % 8 == 0 && p.o_row % 4 == 0 &&
-                  k_range < (std::int64_t{1} << 31) && v_range < (std::int64_t{1} << 31);
-    if (p.int8_operands) {
-        if (!p.fuse_q_quant) vector = vector && aligned(p.Q8, 16);
-        if (p.q8_out) vector = vector && aligned(p.q8_out, 8);
-        vector = vector && aligned(p.K8, 16);
-    }
+    const bool vector = access_piece(p) == 16 && p.o_vector && (!p.q8_out || aligned(p.q8_out, 8)) &&
+                        k_range < (std::int64_t{1} << 31) && v_range < (std::int64_t{1} << 31);
     const int dc = (p.d + 31) / 32;
     switch (dc) {
         case 1: return launch_dc<1>(p, vector, precise, stream);
@@ -1208,15 +1196,17 @@ hipError_t launch_attention(AttnParams p, bool precise, hipStream_t stream) {
 }  // namespace
 }  // namespace tilemix
 
-// Workspace of the per-head entry point's key-range split (partial O rows and
-// row states of every split, [splits][M][d] + [splits][M][2] fp32). One copy
-// per GPU, held until the process ends; the library allocates nothing.
-// Split calls on a device are ordered through one event (each waits for the
-// previous split call's combine, whatever its stream), so concurrent streams
-// never share it at once; calls made while their stream is being captured
-// into a graph take the plain launch instead.
+// Workspace of the key-range splits (partial O rows and row states of every
+// split) and the arrival counters of the decode kernel. One copy per GPU, held
+// until the process ends; the library allocates nothing. Split calls on a
+// device are ordered through one event (each waits for the previous split
+// call's last kernel, whatever its stream), so concurrent streams never share
+// the workspace at once; calls made while their stream is being captured into
+// a graph take an unsplit launch instead.
 static constexpr std::size_t kSplitScratchFloats = std::size_t{8} << 20;  // 32 MiB
+static constexpr std::size_t kSplitArrivals = 1024;
 static __device__ __align__(256) float split_scratch[kSplitScratchFloats];
+static __device__ unsigned split_arrivals[kSplitArrivals];  // zero between launches
 
 namespace tilemix {
 namespace {
@@ -1233,6 +1223,7 @@ constexpr int kMinSplitHead = 8;
 
 struct SplitDevice {
     float* scratch = nullptr;
+    unsigned* arrivals = nullptr;
     hipEvent_t done = nullptr;
     bool recorded = false;
 };
@@ -1263,26 +1254,26 @@ int choose_splits(const AttnParams& p, int compute_units) {
     return splits > 1 ? splits : 1;
 }
 
-// launch_attention, with the key range split over several workgroups per
-// 128-row block when choose_splits says so: the attention kernel writes each
-// split's partial rows to the workspace, split_combine_kernel merges them
-// into O, both on `stream`.
-hipError_t launch_attention_split(AttnParams p, bool precise, hipStream_t stream) {
-    int units = 0;
-    hipError_t status = check_device(&units);
-    if (status != hipSuccess) return status;
-    int splits = choose_splits(p, units);
-    if (splits > 1) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) splits = 1;
-    }
+// The current device's number when a call on `stream` may use the workspace
+// there, -1 when it may not (the stream is being captured, or the device is
+// beyond the table).
+int workspace_device(hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return -1;
     int device = 0;
-    if (splits > 1 && (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)) splits = 1;
-    if (splits <= 1) return launch_attention(p, precise, stream);
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return -1;
+    return device;
+}
 
+// Calls launch(scratch, arrivals), which enqueues kernels on `stream` that use
+// the workspace of `device` (the current one), ordered after the previous
+// call's and before the next one's.
+template <typename Launch>
+hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
     std::lock_guard<std::mutex> guard(split_lock());
     SplitDevice& state = split_devices()[device];
-    if (!state.scratch || !state.done) {
+    hipError_t status = hipSuccess;
+    if (!state.scratch || !state.arrivals || !state.done) {
         // First split call on this device: another thread may be capturing a
         // graph in global mode, which would reject these runtime calls (they
         // enqueue no work), so this thread's capture mode is relaxed around
@@ -1290,12 +1281,16 @@ hipError_t launch_attention_split(AttnParams p, bool precise, hipStream_t stream
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         status = hipThreadExchangeStreamCaptureMode(&mode);
         if (status != hipSuccess) return status;
+        void* address = nullptr;
         if (!state.scratch) {
-            void* address = nullptr;
             status = hipGetSymbolAddress(&address, HIP_SYMBOL(split_scratch));
             if (status == hipSuccess) state.scratch = static_cast<float*>(address);
         }
-        if (status == hipSuccess && !state.done) status = hipEventCreateWithFlags(&state.done, hipEventDisableTiming);
+        if (status == hipSuccess && !state.arrivals) {
+            status = hipGetSymbolAddress(&address, HIP_SYMBOL(split_arrivals));
+            if (status == hipSuccess) state.arrivals = static_cast<unsigned*>(address);
+        }
+        if (status == hipSuccess && !state.done) status = hipEventCreateWithFlags(&state.done, hipEventDisableTiming | hipEventDisableSystemFence);
         const hipError_t restored = hipThreadExchangeStreamCaptureMode(&mode);
         if (status != hipSuccess) return status;
         if (restored != hipSuccess) return restored;
@@ -1304,26 +1299,75 @@ hipError_t launch_attention_split(AttnParams p, bool precise, hipStream_t stream
         status = hipStreamWaitEvent(stream, state.done, 0);
         if (status != hipSuccess) return status;
     }
-    const int tiles = (p.N - 1) / kTileKeys + 1;
-    p.split_tiles = (tiles + splits - 1) / splits;
-    p.splits = (tiles + p.split_tiles - 1) / p.split_tiles;
-    p.part_o = state.scratch;
-    p.part_ml = state.scratch + static_cast<std::size_t>(p.splits) * p.M * p.d;
-    status = launch_attention(p, precise, stream);
-    if (status != hipSuccess) return status;
-    float* const O = static_cast<float*>(p.O);
-    const std::int64_t threads = static_cast<std::int64_t>(p.M) * ((p.d + 3) / 4);
-    const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
-    if (p.d % 4 == 0 && aligned(O, 16) && p.o_row % 4 == 0)
-        split_combine_kernel<true><<<blocks, 256, 0, stream>>>(p.part_o, p.part_ml, p.splits, p.M, p.d, O, p.o_row);
-    else
-        split_combine_kernel<false><<<blocks, 256, 0, stream>>>(p.part_o, p.part_ml, p.splits, p.M, p.d, O, p.o_row);
-    status = hipGetLastError();
+    status = launch(state.scratch, state.arrivals);
     if (status != hipSuccess) return status;
     status = hipEventRecord(state.done, stream);
     if (status != hipSuccess) return status;
     state.recorded = true;
     return hipSuccess;
+}
+
+// launch_attention, with the key range split over several workgroups per
+// 128-row block when choose_splits says so: the attention kernel writes each
+// split's partial rows to the workspace, split_combine_kernel merges them
+// into O, both on `stream`.
+hipError_t launch_attention_split(AttnParams p, bool precise, hipStream_t stream) {
+    int units = 0;
+    const hipError_t found = check_device(&units);
+    if (found != hipSuccess) return found;
+    const int splits = choose_splits(p, units);
+    const int device = splits > 1 ? workspace_device(stream) : -1;
+    if (device < 0) return launch_attention(p, precise, stream);
+    return with_workspace(device, stream, [&](float* scratch, unsigned*) {
+        const int tiles = (p.N - 1) / kTileKeys + 1;
+        p.split_tiles = (tiles + splits - 1) / splits;
+        p.splits = (tiles + p.split_tiles - 1) / p.split_tiles;
+        p.part_o = scratch;
+        p.part_ml = scratch + static_cast<std::size_t>(p.splits) * p.M * p.d;
+        const hipError_t status = launch_attention(p, precise, stream);
+        if (status != hipSuccess) return status;
+        float* const O = static_cast<float*>(p.O);
+        const std::int64_t threads = static_cast<std::int64_t>(p.M) * ((p.d + 3) / 4);
+        const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
+        if (p.d % 4 == 0 && aligned(O, 16) && p.o_row % 4 == 0)
+            split_combine_kernel<true><<<blocks, 256, 0, stream>>>(p.part_o, p.part_ml, p.splits, p.M, p.d, O, p.o_row);
+        else
+            split_combine_kernel<false><<<blocks, 256, 0, stream>>>(p.part_o, p.part_ml, p.splits, p.M, p.d, O, p.o_row);
+        return hipGetLastError();
+    });
+}
+
+// Whether the decode kernel (decode.hip) takes the call: one 16-row cell of
+// queries per head, no causal mask (whose query i sees keys up to i only), and
+// rows that 32-bit buffer offsets reach, up to a step past the last one. At 16
+// rows and below the prefill kernel has query rows for half of one wave of its
+// four. Measured against it, 128 features: 4 heads x 64 keys 9.5 us either
+// way; 32 x 1024 30.1 -> 12.7 us; 32 x 16384 428 -> 54 us. Verification
+// outputs do not change the choice, so they never change O.
+bool decode_ok(const AttnParams& p) {
+    constexpr std::int64_t kReach = std::int64_t{1} << 30;  // halves
+    return p.M <= kMaxDecodeRows && !p.causal && p.q_row * kMaxDecodeRows < kReach &&
+           (p.N + std::int64_t{64}) * p.k_row < kReach && (p.N + std::int64_t{64}) * p.v_row < kReach &&
+           decode_worthwhile(p);
+}
+
+hipError_t launch_decode_split(AttnParams p, bool precise, hipStream_t stream) {
+    int units = 0;
+    const hipError_t found = check_device(&units);
+    if (found != hipSuccess) return found;
+    const int splits = plan_decode(p, units, kSplitScratchFloats, kSplitArrivals);
+    const int device = splits > 1 ? workspace_device(stream) : -1;
+    if (device < 0) return launch_decode(p, 1, precise, stream);
+    return with_workspace(device, stream, [&](float* scratch, unsigned* arrivals) {
+        p.part_o = scratch;
+        p.arrivals = arrivals;
+        return launch_decode(p, splits, precise, stream);
+    });
+}
+
+// O takes whole vector stores: 16-byte fp32 or 8-byte 16-bit pieces of rows.
+int o_vector(const AttnParams& p) {
+    return p.d % 4 == 0 && aligned(p.O, 16) && p.o_stride % 4 == 0 && p.o_row % 4 == 0;
 }
 
 AttnParams base_params(const std::uint16_t* Q, const std::uint16_t* K, const std::uint16_t* V, float* O,
@@ -1390,6 +1434,8 @@ extern "C" int tilemix_attention(const std::uint16_t* Q, const std::uint16_t* K,
     // The per-head API keeps the reference's fp32-level accuracy (its own test
     // suite checks 1e-5 + 1e-4|x| against fp64), so P.V runs in split precision.
     // A head too small to fill the device has its key range split.
+    p.o_vector = o_vector(p);
+    if (decode_ok(p)) return launch_decode_split(p, /*precise=*/true, static_cast<hipStream_t>(stream));
     return launch_attention_split(p, /*precise=*/true, static_cast<hipStream_t>(stream));
 }
 
@@ -1464,6 +1510,8 @@ extern "C" int tilemix_attention_batched(const TileMixBatchedArgs* args, void* s
         p.q8_out = a.Q8;
         p.q_scales_out = a.q_scales;
     }
+    p.o_vector = o_vector(p);
+    if (decode_ok(p)) return launch_decode_split(p, a.precise != 0, static_cast<hipStream_t>(stream));
     return launch_attention(p, a.precise != 0, static_cast<hipStream_t>(stream));
 }
 

@@ -76,6 +76,8 @@ struct AttnParams {
     int split_tiles;
     float* part_o;
     float* part_ml;
+    unsigned* arrivals;  // last_arrival counters, zero between launches
+    int o_vector;        // rows of O take 16-byte (fp32) / 8-byte (16-bit) stores
     // > 0: the workgroups one XCD holds at once (its slots). A head whose
     // query blocks span several rounds of that many workgroups streams its
     // K / V once per round; a workgroup of an odd round walks its key tiles
@@ -247,6 +249,34 @@ __device__ __forceinline__ void set_priority() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Partial results that another workgroup of the launch reads: stores that
+// write through the XCD's L2 to the point where all XCDs agree, and loads that
+// do not take a line the L2 holds (sc1, device scope). A release of ordinary
+// stores would write back the whole L2 instead, once per workgroup: with 512
+// workgroups that measured 25 us more per launch.
+inline constexpr int kDeviceScope = 16;  // sc1 in a buffer instruction's aux operand
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t shared_rows(float* base, std::int64_t floats) {
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(floats * 4), kBufferFlags);
+}
+
+// Whether this workgroup is the last of `count` to arrive at `counter`. The
+// device-scope stores of every wave are complete when it waits for vmcnt(0),
+// before the barrier and the count, so the last workgroup's device-scope loads
+// see all of them. The counter is zero again when the last one has arrived.
+// Every thread of the workgroup calls it; `shared` is a workgroup variable.
+__device__ __forceinline__ bool last_arrival(unsigned* counter, int count, int* shared) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = before == static_cast<unsigned>(count) - 1u;
+        if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *shared = last;
+    }
+    __syncthreads();
+    return *shared != 0;
+}
+
 // Workgroup index -> (head, row group). Workgroups are dealt round-robin to
 // the XCDs; all row groups of a head run on one XCD so that its K / V / K8
 // stay in that XCD's L2. Causal problems take an XCD's heads four at a time
@@ -282,5 +312,40 @@ __device__ __forceinline__ void map_block(int linear, int heads, int groups, boo
 __device__ __forceinline__ bool reversed_round(int linear, int reverse_slots) {
     return reverse_slots > 0 && ((linear / kXcds / reverse_slots) & 1) != 0;
 }
+
+// ---------------------------------------------------------------- host side
+
+inline bool aligned(const void* pointer, std::size_t bytes) {
+    return (reinterpret_cast<std::uintptr_t>(pointer) % bytes) == 0;
+}
+
+// Bytes of the widest contiguous load that every row of Q, K and V (and of Q8
+// and K8 where they are read) allows: 16 for all of them; 8: 16 bytes for the
+// fp16 rows, 4 for the int8 ones (d a multiple of 8, not of 16); 4 for all; 0
+// for single values.
+inline int access_piece(const AttnParams& p) {
+    const bool q8_read = p.int8_operands && !p.fuse_q_quant;
+    auto rows_ok = [&](int halves) {
+        for (const std::int64_t stride : {p.q_stride, p.k_stride, p.v_stride, p.q_row, p.k_row, p.v_row})
+            if (stride % halves != 0) return false;
+        return aligned(p.Q, 2 * halves) && aligned(p.K, 2 * halves) && aligned(p.V, 2 * halves);
+    };
+    auto bytes_ok = [&](int bytes) {
+        return !p.int8_operands || (p.d % bytes == 0 && aligned(p.K8, bytes) && (!q8_read || aligned(p.Q8, bytes)));
+    };
+    if (p.d % 16 == 0 && rows_ok(8) && bytes_ok(16)) return 16;
+    if (p.d % 8 == 0 && rows_ok(8) && bytes_ok(4)) return 8;
+    if (p.d % 4 == 0 && rows_ok(2) && bytes_ok(4)) return 4;
+    return 0;
+}
+
+// decode.hip: M <= kMaxDecodeRows query rows per head. decode_worthwhile:
+// whether it is the faster kernel for the call; plan_decode: workgroups
+// per head for a workspace of scratch_floats and max_arrivals counters (1:
+// none needed); launch_decode with p.part_o and p.arrivals set if splits > 1.
+inline constexpr int kMaxDecodeRows = 16;
+bool decode_worthwhile(const AttnParams& p);
+int plan_decode(const AttnParams& p, int compute_units, std::size_t scratch_floats, std::size_t max_arrivals);
+hipError_t launch_decode(AttnParams p, int splits, bool precise, hipStream_t stream);
 
 }  // namespace tilemix
