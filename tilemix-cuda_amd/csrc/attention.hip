@@ -262,16 +262,24 @@ __device__ __forceinline__ void load_slots(int4v rsrc, unsigned first, const int
     load_slots_from<0, kSlots>(rsrc, first, voffset, soffset);
 }
 
+// kPiece: what rows allow (access_piece). 16: tiles move by LDS DMA in 16-byte
+// pieces. 8 (d a multiple of 8 only): K and V the same way, and K8 rows, which
+// start on 8 bytes, in 16-byte pieces from dword-aligned addresses; a row's
+// last piece may carry the next row's first bytes, which meet zeros of Q8. 4:
+// K and V rows too; what a K row's last piece carries past d is masked when it
+// is read (V's reaches only features past d of O). A piece that would end past
+// the head comes in by dwords instead (load_tile_dwords). 0: single elements.
 // kSplit: the workgroup covers one range of key tiles of its 128-row block
 // and writes that range's partial row state (AttnParams::splits); only the
 // per-head entry point launches it.
-template <int DC, bool kVector, bool kPrecise, bool kDots, bool kSplit>
+template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
 __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kernel(const AttnParams p) {
     using L = Layout<DC>;
     constexpr int kDP = L::kDP;
     constexpr int kOB = DC;               // 32-feature output blocks
     constexpr int kQC = kDP / 16;         // 16-feature Q / K chunks (fp16 MFMA k-steps)
     constexpr int kQ8C = L::kDP8 / 32;    // 32-feature Q8 / K8 chunks (int8 MFMA k-steps)
+    constexpr bool kVector = kPiece >= 8;  // 16-byte pieces of fp16 rows, whole-vector stores
     __shared__ __attribute__((aligned(16))) unsigned char smem[L::kSmemBytes];
     __shared__ unsigned group_bits[kWavesPerGroup];
     // Landing area of the spare DMA slots (written with zeros, never read).
@@ -322,6 +330,13 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 qf[c] = (row < M && feature < d)
                     ? *reinterpret_cast<const half8*>(Qh + static_cast<std::int64_t>(row) * p.q_row + feature)
                     : half8{};
+            } else if constexpr (kPiece == 4) {
+                uint4v words{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    if (row < M && feature + 2 * w < d)
+                        words[w] = *reinterpret_cast<const std::uint32_t*>(Qh + static_cast<std::int64_t>(row) * p.q_row + feature + 2 * w);
+                qf[c] = __builtin_bit_cast(half8, words);
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
@@ -442,10 +457,16 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
             for (int m = 0; m < kQ8C; ++m) {
                 const int feature = 32 * m + 16 * h;
                 int4v chunk;
-                if constexpr (kVector) {
+                if constexpr (kPiece == 16) {
                     chunk = (row < M && feature < d)
                         ? *reinterpret_cast<const int4v*>(Q8h + static_cast<std::int64_t>(row) * d + feature)
                         : int4v{0, 0, 0, 0};
+                } else if constexpr (kPiece != 0) {
+                    chunk = int4v{0, 0, 0, 0};
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        if (row < M && feature + 4 * w < d)
+                            chunk[w] = *reinterpret_cast<const int*>(Q8h + static_cast<std::int64_t>(row) * d + feature + 4 * w);
                 } else {
                     unsigned char bytes[16];
 #pragma unroll
@@ -525,7 +546,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     const unsigned lds_spare_address = lds_address_of(lds_spare);
     int off_k[L::kKPerWave], off_v[L::kVPerWave], off_k8[L::kK8PerWave];
     unsigned dst_k[L::kKPerWave], dst_v[L::kVPerWave], dst_k8[L::kK8PerWave];
-    if constexpr (kVector) {
+    if constexpr (kPiece != 0) {
 #pragma unroll
         for (int t = 0; t < L::kKPerWave; ++t) {
             const int w = wave + kWavesPerGroup * t;
@@ -576,17 +597,38 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 load_to_lds(r, dst_v[t] == lds_spare_address ? dst_v[t] : dst_v[t] + shift, off_v[t], soffset);
         }
     };
+    // A tile whose rows are not whole 16-byte pieces and that reaches the
+    // head's last row (whose last piece would end past the head): dwords
+    // through registers, zeros past d and N. at(row, byte): the LDS position.
+    auto load_tile_dwords = [&](unsigned char* tile, const unsigned char* head_rows, std::int64_t row_bytes, int k0,
+                                int valid_bytes, int padded_bytes, auto&& at) {
+        const int per_row = padded_bytes / 4;
+        for (int e = tid; e < kTileKeys * per_row; e += kThreadsPerGroup) {
+            const int row = e / per_row, byte = 4 * (e % per_row);
+            *reinterpret_cast<std::uint32_t*>(tile + at(row, byte)) =
+                (k0 + row < N && byte < valid_bytes)
+                    ? *reinterpret_cast<const std::uint32_t*>(head_rows + (k0 + row) * row_bytes + byte)
+                    : 0u;
+        }
+    };
     // K (FP16 cells) and K8 (INT8 cells) of tile j.
     auto issue_k = [&](int j, bool need16, bool need8) {
         const int k0 = j * kTileKeys;
-        if constexpr (kVector) {
+        if constexpr (kPiece != 0) {
             const bool tail = k0 + kTileKeys > N;
+            const bool last = k0 + kTileKeys >= N;  // holds the head's last row
             if (need16) {
-                if (tail) k_slots(rsrc_from(rsrc_k, k0 * k_row_bytes), 0);
+                if (kPiece == 4 && last)
+                    load_tile_dwords(lds_k, reinterpret_cast<const unsigned char*>(Kh), p.k_row * 2, k0, 2 * d, 2 * kDP,
+                                     [](int row, int byte) { return L::k_at(row, byte); });
+                else if (tail) k_slots(rsrc_from(rsrc_k, k0 * k_row_bytes), 0);
                 else k_slots(rsrc_k, k0 * k_row_bytes);
             }
             if (need8) {
-                if (tail) k8_slots(rsrc_from(rsrc_k8, k0 * d), 0);
+                if (kPiece != 16 && last)
+                    load_tile_dwords(lds_k8, reinterpret_cast<const unsigned char*>(K8h), d, k0, d, L::kDP8,
+                                     [](int row, int byte) { return L::k8_at(row, byte); });
+                else if (tail) k8_slots(rsrc_from(rsrc_k8, k0 * d), 0);
                 else k8_slots(rsrc_k8, k0 * d);
             }
         } else {
@@ -608,8 +650,11 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     };
     auto issue_v = [&](int j, int buffer) {
         const int k0 = j * kTileKeys;
-        if constexpr (kVector) {
-            if (k0 + kTileKeys > N) v_slots(rsrc_from(rsrc_v, k0 * v_row_bytes), 0, buffer);
+        if constexpr (kPiece != 0) {
+            if (kPiece == 4 && k0 + kTileKeys >= N)
+                load_tile_dwords(lds_v + (buffer ? L::kV1Offset : 0), reinterpret_cast<const unsigned char*>(Vh),
+                                 p.v_row * 2, k0, 2 * d, 2 * kDP, [](int row, int byte) { return L::v_at(row, byte); });
+            else if (k0 + kTileKeys > N) v_slots(rsrc_from(rsrc_v, k0 * v_row_bytes), 0, buffer);
             else v_slots(rsrc_v, k0 * v_row_bytes, buffer);
         } else {
             unsigned char* const dst = lds_v + (buffer ? L::kV1Offset : 0);
@@ -738,8 +783,16 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 half8 kf[3][2];
                 auto load_c = [&](int cc, half8 (&dst)[2]) {
 #pragma unroll
-                    for (int kb = 0; kb < 2; ++kb)
+                    for (int kb = 0; kb < 2; ++kb) {
                         dst[kb] = *reinterpret_cast<const half8*>(lds_k + 32 * L::kKStride * kb + k_lane[cc]);
+                        if constexpr (kPiece == 4) {  // features past d belong to the next row
+                            uint4v words = __builtin_bit_cast(uint4v, dst[kb]);
+#pragma unroll
+                            for (int w = 0; w < 4; ++w)
+                                if (16 * cc + 8 * h + 2 * w >= d) words[w] = 0u;
+                            dst[kb] = __builtin_bit_cast(half8, words);
+                        }
+                    }
                 };
                 load_c(0, kf[0]);
                 load_c(1, kf[1]);
@@ -910,7 +963,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     // 32 rows in kDP / 32 passes of 32 features through a 4 KiB region.
     // out / out_row: the head's first row and the distance between rows, in
     // floats; every value is multiplied by factor.
-    constexpr bool kStaged = kVector && !kDots && (kDP == 128 || kDP == 64);
+    constexpr bool kStaged = kPiece == 16 && !kDots && (kDP == 128 || kDP == 64);
     auto store_staged = [&](float* out, std::int64_t out_row, float factor) {
         if constexpr (kStaged) {
             constexpr int kRowBytes = 128;           // 32 features per pass
@@ -996,7 +1049,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 for (int r4 = 0; r4 < 4; ++r4) {
                     const int feature = (r4 < 2 ? 0 : kDP / 2 - 16) + 16 * fb + 8 * r4 + 4 * h;
                     const float4v value{st.o[fb][4 * r4], st.o[fb][4 * r4 + 1], st.o[fb][4 * r4 + 2], st.o[fb][4 * r4 + 3]};
-                    store_output(part, TILEMIX_DTYPE_F32, row_offset + feature, value, d - feature, kVector);
+                    store_output(part, TILEMIX_DTYPE_F32, row_offset + feature, value, d - feature, kPiece != 0);
                 }
             if (h == 0) {
                 float* const ml = p.part_ml + 2 * (static_cast<std::int64_t>(split) * M + row);
@@ -1026,7 +1079,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                     // 16 fb + R (R < 16) or kDP / 2 + 16 fb + R - 16.
                     const int feature = (r4 < 2 ? 0 : kDP / 2 - 16) + 16 * fb + 8 * r4 + 4 * h;
                     const float4v value{st.o[fb][4 * r4], st.o[fb][4 * r4 + 1], st.o[fb][4 * r4 + 2], st.o[fb][4 * r4 + 3]};
-                    store_output(Oh, p.o_dtype, row_offset + feature, value * inverse, d - feature, kVector);
+                    store_output(Oh, p.o_dtype, row_offset + feature, value * inverse, d - feature, kVector || p.o_vector);
                 }
         }
     }
@@ -1093,34 +1146,37 @@ __global__ __launch_bounds__(256) void split_combine_kernel(const float* part_o,
     }
 }
 
-template <int DC, bool kVector, bool kPrecise, bool kDots, bool kSplit>
+template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
 hipError_t launch_variant(const AttnParams& p, hipStream_t stream) {
     const unsigned blocks = static_cast<unsigned>(p.q_blocks) * static_cast<unsigned>(p.heads) *
                             static_cast<unsigned>(kSplit ? p.splits : 1);
-    attention_kernel<DC, kVector, kPrecise, kDots, kSplit><<<blocks, kThreadsPerGroup, 0, stream>>>(p);
+    attention_kernel<DC, kPiece, kPrecise, kDots, kSplit><<<blocks, kThreadsPerGroup, 0, stream>>>(p);
     return hipGetLastError();
 }
 
 // Split launches exist for the per-head entry point only, whose P.V is
 // always the precise one.
-template <int DC, bool kVector>
-hipError_t launch_vp(const AttnParams& p, bool precise, bool dots, hipStream_t stream) {
+template <int DC, int kPiece, bool kDots>
+hipError_t launch_vp(const AttnParams& p, bool precise, hipStream_t stream) {
     if (p.splits > 1) {
         if (!precise) return hipErrorInvalidValue;
-        return dots ? launch_variant<DC, kVector, true, true, true>(p, stream)
-                    : launch_variant<DC, kVector, true, false, true>(p, stream);
+        return launch_variant<DC, kPiece, true, kDots, true>(p, stream);
     }
-    if (precise)
-        return dots ? launch_variant<DC, kVector, true, true, false>(p, stream)
-                    : launch_variant<DC, kVector, true, false, false>(p, stream);
-    return dots ? launch_variant<DC, kVector, false, true, false>(p, stream)
-                : launch_variant<DC, kVector, false, false, false>(p, stream);
+    return precise ? launch_variant<DC, kPiece, true, kDots, false>(p, stream)
+                   : launch_variant<DC, kPiece, false, kDots, false>(p, stream);
 }
 
+// Verification outputs (dots, trace) take the 16-byte or the element kernel.
 template <int DC>
-hipError_t launch_dc(const AttnParams& p, bool vector, bool precise, hipStream_t stream) {
-    const bool dots = p.dots != nullptr || p.trace != nullptr;
-    return vector ? launch_vp<DC, true>(p, precise, dots, stream) : launch_vp<DC, false>(p, precise, dots, stream);
+hipError_t launch_dc(const AttnParams& p, int piece, bool precise, hipStream_t stream) {
+    if (p.dots != nullptr || p.trace != nullptr)
+        return piece == 16 ? launch_vp<DC, 16, true>(p, precise, stream) : launch_vp<DC, 0, true>(p, precise, stream);
+    switch (piece) {
+        case 16: return launch_vp<DC, 16, false>(p, precise, stream);
+        case 8: return launch_vp<DC, 8, false>(p, precise, stream);
+        case 4: return launch_vp<DC, 4, false>(p, precise, stream);
+        default: return launch_vp<DC, 0, false>(p, precise, stream);
+    }
 }
 
 std::size_t words_per_row(int N, int group) {
@@ -1178,18 +1234,22 @@ hipError_t launch_attention(AttnParams p, bool precise, hipStream_t stream) {
     const int xcd_slots = units / kXcds * kGroupsPerCU;
     p.reverse_slots = (!p.causal && p.splits <= 1 && p.heads % kXcds == 0 && xcd_slots > 0 && p.q_blocks > xcd_slots)
                           ? xcd_slots : 0;
-    // The vector path moves 16-byte pieces and addresses a head's K / V with
-    // 32-bit buffer offsets; other shapes take the element-wise path.
+    // DMA paths address a head's K / V with 32-bit buffer offsets; longer
+    // heads take the element-wise path. The 16-byte store forms need aligned
+    // rows of O (and 8-byte ones of Q8); without them the dword form, which
+    // picks its stores at run time, takes the call. Measured (12 heads x 1003
+    // x 72, causal, precise P.V): 300 us with elements, 42.6 with pieces; d = 100
+    // 347 and 68.7.
     const std::int64_t k_range = (static_cast<std::int64_t>(p.N - 1) * p.k_row + p.d) * 2;
     const std::int64_t v_range = (static_cast<std::int64_t>(p.N - 1) * p.v_row + p.d) * 2;
-    const bool vector = access_piece(p) == 16 && p.o_vector && (!p.q8_out || aligned(p.q8_out, 8)) &&
-                        k_range < (std::int64_t{1} << 31) && v_range < (std::int64_t{1} << 31);
+    int piece = k_range < (std::int64_t{1} << 31) && v_range < (std::int64_t{1} << 31) ? access_piece(p) : 0;
+    if (piece >= 8 && !(p.o_vector && (!p.q8_out || aligned(p.q8_out, 8)))) piece = 4;
     const int dc = (p.d + 31) / 32;
     switch (dc) {
-        case 1: return launch_dc<1>(p, vector, precise, stream);
-        case 2: return launch_dc<2>(p, vector, precise, stream);
-        case 3: return launch_dc<3>(p, vector, precise, stream);
-        default: return launch_dc<4>(p, vector, precise, stream);
+        case 1: return launch_dc<1>(p, piece, precise, stream);
+        case 2: return launch_dc<2>(p, piece, precise, stream);
+        case 3: return launch_dc<3>(p, piece, precise, stream);
+        default: return launch_dc<4>(p, piece, precise, stream);
     }
 }
 
