@@ -68,6 +68,8 @@ int tilemix_quantize_qk(const uint16_t* Q, const uint16_t* K, int8_t* Q8, int8_t
  * second kernel on `stream`. Split calls on one device are ordered through one event (each
  * waits for the previous one's merge, on any stream); a call made while
  * `stream` is being captured into a graph takes the unsplit launch.
+ * tilemix_attention_batched splits a call of few, long row blocks (at least 16
+ * key tiles) in the same way where that saves time.
  * A call of M <= 16 query rows (here and in tilemix_attention_batched without
  * a causal mask) is served by a kernel of its own, which splits the keys of
  * its heads over workgroups of the same launch through the same workspace,

@@ -44,8 +44,10 @@ DEVICE_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-LIB_SOURCES = ["quantize.hip", "attention.hip", "decode.hip", "routing.hip"]
-SOURCE_FLAGS: dict[str, list[str]] = {}
+# (source, object, extra flags): the attention kernels are compiled once per
+# head-dimension class, in parallel.
+LIB_UNITS = [("attention.hip", f"attention_dc{dc}.o", [f"-DTILEMIX_DC={dc}"]) for dc in (4, 3, 2, 1)] + [
+    (name, name + ".o", []) for name in ("decode.hip", "attention.hip", "quantize.hip", "routing.hip")]
 
 
 def _run(cmd: list[str]) -> None:
@@ -60,9 +62,9 @@ def _run(cmd: list[str]) -> None:
         print(err, file=sys.stderr)
 
 
-def compile_object(source: Path, obj: Path) -> Path:
+def compile_object(source: Path, obj: Path, flags: list[str]) -> Path:
     obj.parent.mkdir(parents=True, exist_ok=True)
-    _run([HIPCC, *DEVICE_FLAGS, *SOURCE_FLAGS.get(source.name, []), f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(source),
+    _run([HIPCC, *DEVICE_FLAGS, *flags, f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(source),
           "-o", str(obj)])
     return obj
 
@@ -70,7 +72,7 @@ def compile_object(source: Path, obj: Path) -> Path:
 def build_library(jobs: int) -> Path:
     BUILD.mkdir(parents=True, exist_ok=True)
     with futures.ThreadPoolExecutor(max_workers=jobs) as pool:
-        objects = list(pool.map(lambda s: compile_object(CSRC / s, BUILD / (s + ".o")), LIB_SOURCES))
+        objects = list(pool.map(lambda unit: compile_object(CSRC / unit[0], BUILD / unit[1], unit[2]), LIB_UNITS))
     tmp = LIBRARY.with_suffix(".so.tmp")
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)])
     os.replace(tmp, LIBRARY)

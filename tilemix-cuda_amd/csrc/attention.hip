@@ -178,7 +178,7 @@ struct RowState {
 };
 
 // Maximum of the 16 values of a 32x32 accumulator block, 8 v_max3.
-__device__ __forceinline__ float block_max16(const float16v& x) {
+[[maybe_unused]] __device__ __forceinline__ float block_max16(const float16v& x) {
     const float a = max3(x[0], x[1], x[2]), b = max3(x[3], x[4], x[5]), e = max3(x[6], x[7], x[8]);
     const float f = max3(x[9], x[10], x[11]), g = max3(x[12], x[13], x[14]);
     return max3(max3(a, b, e), max3(f, g, x[15]), x[15]);
@@ -270,8 +270,7 @@ __device__ __forceinline__ void load_slots(int4v rsrc, unsigned first, const int
 // is read (V's reaches only features past d of O). A piece that would end past
 // the head comes in by dwords instead (load_tile_dwords). 0: single elements.
 // kSplit: the workgroup covers one range of key tiles of its 128-row block
-// and writes that range's partial row state (AttnParams::splits); only the
-// per-head entry point launches it.
+// and writes that range's partial row state (AttnParams::splits).
 template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
 __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kernel(const AttnParams p) {
     using L = Layout<DC>;
@@ -310,6 +309,15 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     const int q0 = qblock * kRowsPerGroup;
     const int qw = q0 + wave * kRowsPerWave;
     const int M = p.M, N = p.N, d = p.d;
+    const std::int64_t part = kSplit ? (head * p.splits + split) * M : 0;  // this split's first partial row
+    if constexpr (kSplit && !kDots) {
+        // A range that lies past the block's causal diagonal: no key.
+        if (p.causal && split * p.split_tiles * kTileKeys > q0 + kRowsPerGroup - 1) {
+            if (tid < kRowsPerGroup && q0 + tid < M)
+                *reinterpret_cast<float2v*>(p.part_ml + 2 * (part + q0 + tid)) = float2v{-INFINITY, 0.0f};
+            return;
+        }
+    }
 
     const std::uint16_t* Qh = p.Q + head * p.q_stride;
     const std::uint16_t* Kh = p.K + head * p.k_stride;
@@ -392,7 +400,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
             const float recip = 1.0f / scale;
             const _Float16 stored = static_cast<_Float16>(scale);
             q_scale = static_cast<float>(stored);
-            if (tid == 0 && p.q_scales_out)
+            if (tid == 0 && p.q_scales_out && split == 0)
                 p.q_scales_out[head * p.q_blocks + qblock] = __builtin_bit_cast(std::uint16_t, stored);
             {
                 const int row = qw + q;
@@ -413,7 +421,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                         packed[c][1] = pack_bytes(v[4], v[5], v[6], v[7]);
                     }
                     const int feature = 16 * c + 8 * h;
-                    if (p.q8_out && row < M && feature < d) {
+                    if (p.q8_out && split == 0 && row < M && feature < d) {
                         std::int8_t* dst = p.q8_out + head * static_cast<std::int64_t>(M) * d +
                                            static_cast<std::int64_t>(row) * d + feature;
                         if constexpr (kVector) {
@@ -941,9 +949,11 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         v_buffer ^= 1;
     }
 
-    // Routing trace of tiles a causal workgroup never visits.
-    if (kDots && !kSplit && p.trace && tiles < key_tiles64) {
-        for (int j = tiles; j < key_tiles64; ++j) {
+    // Routing trace of tiles a causal workgroup never visits (of its range, the
+    // last one's to the end).
+    if (kDots && p.trace && p.causal) {
+        const int range_end = kSplit && split + 1 < p.splits ? min(key_tiles64, tile_begin + p.split_tiles) : key_tiles64;
+        for (int j = tiles; j < range_end; ++j) {
             std::uint32_t int8_mask = 0, skip_mask = 0;
             tile_masks(j, int8_mask, skip_mask);
             write_trace(j, int8_mask, skip_mask);
@@ -1031,9 +1041,9 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         const int row = qw + q;
         if constexpr (kStaged) {
             if (d == kDP) {
-                store_staged(p.part_o + static_cast<std::int64_t>(split) * M * d, d, 1.0f);
+                store_staged(p.part_o + part * d, d, 1.0f);
                 if (row < M && h == 0) {
-                    float* const ml = p.part_ml + 2 * (static_cast<std::int64_t>(split) * M + row);
+                    float* const ml = p.part_ml + 2 * (part + row);
                     ml[0] = st.m;
                     ml[1] = a + b;
                 }
@@ -1041,7 +1051,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
             }
         }
         if (row < M) {
-            unsigned char* const part = reinterpret_cast<unsigned char*>(p.part_o + static_cast<std::int64_t>(split) * M * d);
+            unsigned char* const part_rows = reinterpret_cast<unsigned char*>(p.part_o + part * d);
             const std::int64_t row_offset = static_cast<std::int64_t>(row) * d;
 #pragma unroll
             for (int fb = 0; fb < kOB; ++fb)
@@ -1049,10 +1059,10 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 for (int r4 = 0; r4 < 4; ++r4) {
                     const int feature = (r4 < 2 ? 0 : kDP / 2 - 16) + 16 * fb + 8 * r4 + 4 * h;
                     const float4v value{st.o[fb][4 * r4], st.o[fb][4 * r4 + 1], st.o[fb][4 * r4 + 2], st.o[fb][4 * r4 + 3]};
-                    store_output(part, TILEMIX_DTYPE_F32, row_offset + feature, value, d - feature, kPiece != 0);
+                    store_output(part_rows, TILEMIX_DTYPE_F32, row_offset + feature, value, d - feature, kPiece != 0);
                 }
             if (h == 0) {
-                float* const ml = p.part_ml + 2 * (static_cast<std::int64_t>(split) * M + row);
+                float* const ml = p.part_ml + 2 * (part + row);
                 ml[0] = st.m;
                 ml[1] = a + b;
             }
@@ -1087,22 +1097,25 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
 
 // O of a key-range split launch: per row, m = max over the splits of m_s,
 // O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s (log2-domain row states;
-// splits whose rows saw no key have m_s = -inf and weigh nothing). One
-// thread per row and 4 features, splits summed in order. Splits are taken
-// kBatch at a time, every load of a batch issued before any use (one memory
-// round trip per batch); m is the maximum over the splits seen so far, and a
-// later batch that raises it rescales the sums (up to kBatch splits: one
-// batch, m over all splits).
+// splits whose rows saw no key have m_s = -inf and weigh nothing; of those
+// past a causal diagonal only the row states are written). One thread per
+// head, row and 4 features, splits summed in order. Splits are taken kBatch at
+// a time, every load of a batch issued before any use (one memory round trip
+// per batch); m is the maximum over the splits seen so far, and a later batch
+// that raises it rescales the sums (up to kBatch splits: one batch, m over all
+// splits).
 template <bool kVector>
-__global__ __launch_bounds__(256) void split_combine_kernel(const float* part_o, const float* part_ml, int splits,
-                                                           int M, int d, float* O, std::int64_t o_row) {
+__global__ __launch_bounds__(256) void split_combine_kernel(const AttnParams p) {
     constexpr int kBatch = 16;
+    const int M = p.M, d = p.d, splits = p.splits;
     const int groups = (d + 3) / 4;
     const std::int64_t index = static_cast<std::int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (index >= static_cast<std::int64_t>(M) * groups) return;
-    const int row = static_cast<int>(index / groups);
-    const int f0 = 4 * static_cast<int>(index - static_cast<std::int64_t>(row) * groups);
-    const float2v* const ml = reinterpret_cast<const float2v*>(part_ml);
+    const std::int64_t head_row = index / groups;
+    if (head_row >= static_cast<std::int64_t>(p.heads) * M) return;
+    const std::int64_t head = head_row / M;
+    const int row = static_cast<int>(head_row - head * M);
+    const int f0 = 4 * static_cast<int>(index - head_row * groups);
+    const float2v* const ml = reinterpret_cast<const float2v*>(p.part_ml);
     float m = -INFINITY, l = 0.0f;
     float4v acc{0.0f, 0.0f, 0.0f, 0.0f};
     for (int s0 = 0; s0 < splits; s0 += kBatch) {
@@ -1110,9 +1123,9 @@ __global__ __launch_bounds__(256) void split_combine_kernel(const float* part_o,
         float4v value[kBatch];
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
-            const std::int64_t r = static_cast<std::int64_t>(s0 + b < splits ? s0 + b : s0) * M + row;
+            const std::int64_t r = (head * splits + (s0 + b < splits ? s0 + b : s0)) * M + row;
             state[b] = ml[r];
-            const float* src = part_o + r * d + f0;
+            const float* src = p.part_o + r * d + f0;
             if constexpr (kVector) {
                 value[b] = *reinterpret_cast<const float4v*>(src);
             } else {
@@ -1132,18 +1145,16 @@ __global__ __launch_bounds__(256) void split_combine_kernel(const float* part_o,
         }
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
-            const float w = (s0 + b >= splits || state[b][0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(state[b][0] - m);
+            const bool counts = s0 + b < splits && state[b][0] != -INFINITY;
+            const float w = counts ? __builtin_amdgcn_exp2f(state[b][0] - m) : 0.0f;
             l += w * state[b][1];
-            acc += w * value[b];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += w * (counts ? value[b][e] : 0.0f);
         }
     }
     const float inverse = l > 0.0f ? 1.0f / l : 0.0f;
-    float* dst = O + static_cast<std::int64_t>(row) * o_row + f0;
-    if constexpr (kVector) {
-        *reinterpret_cast<float4v*>(dst) = acc * inverse;
-    } else {
-        for (int e = 0; e < 4 && f0 + e < d; ++e) dst[e] = acc[e] * inverse;
-    }
+    unsigned char* const Oh = static_cast<unsigned char*>(p.O) + head * p.o_stride * (p.o_dtype == TILEMIX_DTYPE_F32 ? 4 : 2);
+    store_output(Oh, p.o_dtype, static_cast<std::int64_t>(row) * p.o_row + f0, acc * inverse, d - f0, p.o_vector != 0);
 }
 
 template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
@@ -1154,19 +1165,20 @@ hipError_t launch_variant(const AttnParams& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Split launches exist for the per-head entry point only, whose P.V is
-// always the precise one.
 template <int DC, int kPiece, bool kDots>
 hipError_t launch_vp(const AttnParams& p, bool precise, hipStream_t stream) {
-    if (p.splits > 1) {
-        if (!precise) return hipErrorInvalidValue;
-        return launch_variant<DC, kPiece, true, kDots, true>(p, stream);
-    }
+    if (p.splits > 1)
+        return precise ? launch_variant<DC, kPiece, true, kDots, true>(p, stream)
+                       : launch_variant<DC, kPiece, false, kDots, true>(p, stream);
     return precise ? launch_variant<DC, kPiece, true, kDots, false>(p, stream)
                    : launch_variant<DC, kPiece, false, kDots, false>(p, stream);
 }
 
+}  // namespace
+
 // Verification outputs (dots, trace) take the 16-byte or the element kernel.
+// Each head-dimension class DC is compiled in a unit of its own (TILEMIX_DC,
+// set by the build), in parallel; the unit without it holds the host side.
 template <int DC>
 hipError_t launch_dc(const AttnParams& p, int piece, bool precise, hipStream_t stream) {
     if (p.dots != nullptr || p.trace != nullptr)
@@ -1178,6 +1190,17 @@ hipError_t launch_dc(const AttnParams& p, int piece, bool precise, hipStream_t s
         default: return launch_vp<DC, 0, false>(p, precise, stream);
     }
 }
+
+#ifdef TILEMIX_DC
+template hipError_t launch_dc<TILEMIX_DC>(const AttnParams&, int, bool, hipStream_t);
+}  // namespace tilemix
+#else
+extern template hipError_t launch_dc<1>(const AttnParams&, int, bool, hipStream_t);
+extern template hipError_t launch_dc<2>(const AttnParams&, int, bool, hipStream_t);
+extern template hipError_t launch_dc<3>(const AttnParams&, int, bool, hipStream_t);
+extern template hipError_t launch_dc<4>(const AttnParams&, int, bool, hipStream_t);
+
+namespace {
 
 std::size_t words_per_row(int N, int group) {
     const std::size_t key_tiles = (static_cast<std::size_t>(N) - 1) / kCellKeys + 1;
@@ -1271,15 +1294,43 @@ static __device__ unsigned split_arrivals[kSplitArrivals];  // zero between laun
 namespace tilemix {
 namespace {
 
-// A split covers at least this many key tiles, and a head with fewer than
-// kMinSplitHead key tiles is not split: the split's fixed cost (partial rows,
+// A split covers at least `tiles` key tiles, and a call whose longest row block
+// has fewer than `longest` is not split: the split's fixed cost (partial rows,
 // the combine launch, the ordering event) is about that of a few tiles'
-// walk. Measured per call (M = 4096, d = 128): at N = 256 the plain launch
-// is 23 % faster than two splits; at N = 512 four 2-tile splits are 14 %
-// faster than two 4-tile ones, and the reference demo (16 tiles) 7 % with 8
-// splits than with 4; from N = 4096 on the slot count limits the splits.
-constexpr int kMinSplitTiles = 2;
-constexpr int kMinSplitHead = 8;
+// walk. Measured per call, per-head API (M = 4096, d = 128): at N = 256 the
+// plain launch is 23 % faster than two splits; at N = 512 four 2-tile splits
+// are 14 % faster than two 4-tile ones, and the reference demo (16 tiles) 7 %
+// with 8 splits than with 4; from N = 4096 on the slot count limits the splits.
+// Batched calls are split where split_pays says so.
+// Unsplit | splits of at least 2, 4, 8 tiles (us): 4 heads x 512 x 512 x 64
+// 16.1 | 18.7, 19.8, -; 4 x 2048 causal x 128 46.5 | 26.1, 26.0, 28.2; 16 x
+// 128 x 4096 x 128 80.4 | 32.3, 28.7, 31.6; 8 x 512 x 8192 x 128 168.6 | 36.4,
+// 35.1, 35.0.
+struct SplitRule {
+    int tiles;
+    int longest;
+    bool weigh;
+};
+constexpr SplitRule kSplitHead{2, 8, false};
+constexpr SplitRule kSplitBatch{4, 16, true};
+
+// Whether a split saves more than it costs, from the calls measured above and
+// below. A lone workgroup of a CU walks a tile in about 0.5 + d / 160 us (half
+// as much again with precise P.V, a quarter with routes and no skipped tiles),
+// two walk 9 % slower each; a split costs 4.5 us for the second kernel and the
+// event, and 0.75 us per MB of partial rows, written and read. Unsplit and
+// split, both sides of the line (us): 4 heads x 1024 x 64 20.3, 15.3; 12 x 1003
+// causal x 72 precise 42.6, 31.2; 8 x 2048 causal x 128 52.9, 49.4; 4 x 4096
+// causal x 128 87.5, 56.0 | 32 x 1024 x 64 21.2, 34.8; 16 x 2048 x 64 37.2,
+// 45.9; 16 x 1024 causal x 128 26.6, 34.7; 200 x 64 x 1500 x 64 three-way
+// 40.7, 42.1.
+bool split_pays(const AttnParams& p, bool precise, std::int64_t longest, std::int64_t split_tiles) {
+    const std::int64_t splits = (longest + split_tiles - 1) / split_tiles;
+    const double tile_us = (0.5 + p.d / 160.0) * (precise ? 1.5 : 1.0) * (p.route_words && !p.skip_words ? 1.25 : 1.0);
+    const double saved_us = (longest - 1.09 * split_tiles) * tile_us;
+    const double partial_mb = 4e-6 * static_cast<double>(splits) * p.heads * p.M * (p.d + 2);
+    return saved_us > 1.05 * (4.5 + 0.75 * partial_mb);
+}
 
 struct SplitDevice {
     float* scratch = nullptr;
@@ -1298,20 +1349,35 @@ SplitDevice* split_devices() {
     return devices;
 }
 
-// Key-range splits for a single-head, non-causal launch of at least
-// kMinSplitHead key tiles that would fill less than half of the device's
-// workgroup slots: as many as bring it to one wave of workgroups, each
-// covering at least kMinSplitTiles key tiles and all fitting in the
-// workspace (1 = no split).
-int choose_splits(const AttnParams& p, int compute_units) {
-    if (compute_units <= 0 || p.heads != 1 || p.causal) return 1;
-    const int resident = compute_units * kGroupsPerCU;
-    if (2 * p.q_blocks > resident) return 1;
-    const int tiles = (p.N - 1) / kTileKeys + 1;
-    if (tiles < kMinSplitHead) return 1;
-    int splits = std::min(resident / p.q_blocks, tiles / kMinSplitTiles);
-    while (splits > 1 && static_cast<std::size_t>(splits) * p.M * (p.d + 2) > kSplitScratchFloats) --splits;
-    return splits > 1 ? splits : 1;
+// Key tiles of one split of a launch whose workgroups would fill less than
+// half of the device's slots: as few as spread all tiles over one wave of
+// workgroups, at least the rule's, and enough that the partial rows fit in the
+// workspace (0 = no split).
+int choose_split_tiles(const AttnParams& p, bool precise, int compute_units, const SplitRule& rule) {
+    const std::int64_t resident = static_cast<std::int64_t>(compute_units) * kGroupsPerCU;
+    const std::int64_t items = static_cast<std::int64_t>(p.heads) * p.q_blocks;
+    if (compute_units <= 0 || 2 * items > resident) return 0;
+    const std::int64_t tiles = (p.N - 1) / kTileKeys + 1;
+    std::int64_t longest = tiles, total = items * tiles;
+    if (p.causal) {
+        constexpr int kTilesPerBlock = kRowsPerGroup / kTileKeys;
+        longest = std::min<std::int64_t>(tiles, static_cast<std::int64_t>(kTilesPerBlock) * p.q_blocks);
+        total = 0;
+        for (int block = 0; block < p.q_blocks; ++block) total += std::min<std::int64_t>(tiles, (block + 1) * kTilesPerBlock);
+        total *= p.heads;
+    }
+    if (longest < rule.longest) return 0;
+    std::int64_t split_tiles;
+    if (p.causal) {
+        split_tiles = std::max<std::int64_t>((total + resident - 1) / resident, rule.tiles);
+    } else {
+        const std::int64_t splits = std::max<std::int64_t>(std::min(resident / items, tiles / rule.tiles), 1);
+        split_tiles = (tiles + splits - 1) / splits;
+    }
+    const std::size_t row_floats = static_cast<std::size_t>(p.heads) * p.M * (p.d + 2);
+    while (split_tiles < longest && (longest + split_tiles - 1) / split_tiles * row_floats > kSplitScratchFloats) ++split_tiles;
+    if (split_tiles >= longest || (rule.weigh && !split_pays(p, precise, longest, split_tiles))) return 0;
+    return static_cast<int>(split_tiles);
 }
 
 // The current device's number when a call on `stream` may use the workspace
@@ -1368,31 +1434,31 @@ hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
 }
 
 // launch_attention, with the key range split over several workgroups per
-// 128-row block when choose_splits says so: the attention kernel writes each
-// split's partial rows to the workspace, split_combine_kernel merges them
+// 128-row block when choose_split_tiles says so: the attention kernel writes
+// each split's partial rows to the workspace, split_combine_kernel merges them
 // into O, both on `stream`.
-hipError_t launch_attention_split(AttnParams p, bool precise, hipStream_t stream) {
+hipError_t launch_attention_split(AttnParams p, bool precise, const SplitRule& rule, hipStream_t stream) {
     int units = 0;
     const hipError_t found = check_device(&units);
     if (found != hipSuccess) return found;
-    const int splits = choose_splits(p, units);
-    const int device = splits > 1 ? workspace_device(stream) : -1;
+    const int split_tiles = choose_split_tiles(p, precise, units, rule);
+    const int device = split_tiles > 0 ? workspace_device(stream) : -1;
     if (device < 0) return launch_attention(p, precise, stream);
     return with_workspace(device, stream, [&](float* scratch, unsigned*) {
-        const int tiles = (p.N - 1) / kTileKeys + 1;
-        p.split_tiles = (tiles + splits - 1) / splits;
-        p.splits = (tiles + p.split_tiles - 1) / p.split_tiles;
+        int tiles = (p.N - 1) / kTileKeys + 1;
+        if (p.causal) tiles = std::min(tiles, p.q_blocks * (kRowsPerGroup / kTileKeys));
+        p.split_tiles = split_tiles;
+        p.splits = (tiles + split_tiles - 1) / split_tiles;
         p.part_o = scratch;
-        p.part_ml = scratch + static_cast<std::size_t>(p.splits) * p.M * p.d;
+        p.part_ml = scratch + static_cast<std::size_t>(p.heads) * p.splits * p.M * p.d;
         const hipError_t status = launch_attention(p, precise, stream);
         if (status != hipSuccess) return status;
-        float* const O = static_cast<float*>(p.O);
-        const std::int64_t threads = static_cast<std::int64_t>(p.M) * ((p.d + 3) / 4);
+        const std::int64_t threads = static_cast<std::int64_t>(p.heads) * p.M * ((p.d + 3) / 4);
         const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
-        if (p.d % 4 == 0 && aligned(O, 16) && p.o_row % 4 == 0)
-            split_combine_kernel<true><<<blocks, 256, 0, stream>>>(p.part_o, p.part_ml, p.splits, p.M, p.d, O, p.o_row);
+        if (p.d % 4 == 0)
+            split_combine_kernel<true><<<blocks, 256, 0, stream>>>(p);
         else
-            split_combine_kernel<false><<<blocks, 256, 0, stream>>>(p.part_o, p.part_ml, p.splits, p.M, p.d, O, p.o_row);
+            split_combine_kernel<false><<<blocks, 256, 0, stream>>>(p);
         return hipGetLastError();
     });
 }
@@ -1496,7 +1562,7 @@ extern "C" int tilemix_attention(const std::uint16_t* Q, const std::uint16_t* K,
     // A head too small to fill the device has its key range split.
     p.o_vector = o_vector(p);
     if (decode_ok(p)) return launch_decode_split(p, /*precise=*/true, static_cast<hipStream_t>(stream));
-    return launch_attention_split(p, /*precise=*/true, static_cast<hipStream_t>(stream));
+    return launch_attention_split(p, /*precise=*/true, kSplitHead, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tilemix_attention_batched(const TileMixBatchedArgs* args, void* stream) {
@@ -1572,7 +1638,7 @@ extern "C" int tilemix_attention_batched(const TileMixBatchedArgs* args, void* s
     }
     p.o_vector = o_vector(p);
     if (decode_ok(p)) return launch_decode_split(p, a.precise != 0, static_cast<hipStream_t>(stream));
-    return launch_attention(p, a.precise != 0, static_cast<hipStream_t>(stream));
+    return launch_attention_split(p, a.precise != 0, kSplitBatch, static_cast<hipStream_t>(stream));
 }
 
 extern "C" std::size_t tilemix_routing_words_per_row_c(int N, int key_tiles_per_group) {
@@ -1591,3 +1657,4 @@ extern "C" std::size_t tilemix_shared_bytes_c(int d, int quantized) {
 }
 
 extern "C" const char* tilemix_version(void) { return "tilemix-hip 0.1 gfx950"; }
+#endif  // TILEMIX_DC
