@@ -58,6 +58,7 @@
 #include <cmath>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 namespace tilemix {
 namespace {
@@ -189,7 +190,7 @@ struct RowState {
 // pass c = 1). ph[ks] / pl[ks] receive the fp16 probabilities of keys
 // 16 ks + {4h .. 4h + 3, 8 + 4h .. 8 + 4h + 3}: the B operand (P^T) of the
 // 32x32x16 P.V MFMA for key step ks.
-template <int kOB, bool kPrecise>
+template <int kOB, bool kPrecise, bool kPriority = true>
 __device__ __forceinline__ void softmax_tile(RowState<kOB>& st, const float16v (&x)[2], float c,
                                              half8 (&ph)[4], half8 (&pl)[4]) {
     const float tile = max3(block_max16(x[0]), block_max16(x[1]), block_max16(x[1])) * c;  // c >= 0
@@ -228,7 +229,7 @@ __device__ __forceinline__ void softmax_tile(RowState<kOB>& st, const float16v (
             if constexpr (kPrecise) sum = __builtin_amdgcn_fdot2(half2v{pl[ks][e], pl[ks][e + 1]}, ones, sum, false);
         }
         part[ks] = sum;
-        if (ks == 1) set_priority<2>();  // second half of the VALU phase
+        if (kPriority && ks == 1) set_priority<2>();  // second half of the VALU phase
     }
     st.lsum += (part[0] + part[1]) + (part[2] + part[3]);
 }
@@ -260,6 +261,254 @@ __device__ __forceinline__ void load_slots_from(int4v rsrc, unsigned first, cons
 template <int kSlots>
 __device__ __forceinline__ void load_slots(int4v rsrc, unsigned first, const int (&voffset)[kSlots], int soffset) {
     load_slots_from<0, kSlots>(rsrc, first, voffset, soffset);
+}
+
+// The pieces one of eight waves moves of a tile buffer kBase bytes past the
+// wave's first LDS address: slot t lands 8 KiB past slot t - 1. `base` bytes
+// are added to the lanes' offsets, so the range check covers the whole address.
+template <int kBase, int t, int kSlots>
+__device__ __forceinline__ void load_slots_at(int4v rsrc, unsigned first, const int (&voffset)[kSlots], int base) {
+    if constexpr (t < kSlots) {
+        load_to_lds_at<kBase + 8192 * t>(rsrc, first, voffset[t] + base, 0);
+        load_slots_at<kBase, t + 1, kSlots>(rsrc, first, voffset, base);
+    }
+}
+
+// fp32 rows of 128 or 64 features (O, or a split's partial rows) leave the
+// kernels without dot export through LDS. From registers, each store
+// instruction writes 16 bytes to each of 32 rows, i.e. 32 partial cache lines,
+// and those lines, held in the XCD's L2 until written back, evict K / V tiles.
+// Staged, each store writes 8 rows x 128 bytes (full cache lines) with a
+// non-temporal hint, so the rows bypass the L2. Each wave stages its 32 rows
+// (qw .. qw + 31 of M) in kOB passes of 32 features through its own region of
+// kStageBytes, which no other wave or load uses. out / out_row: the head's
+// first row and the distance between rows, in floats; every value is
+// multiplied by factor.
+constexpr int kStageBytes = 32 * 128;
+template <int kOB>
+__device__ __forceinline__ void store_staged(const RowState<kOB>& st, unsigned char* region, float* out,
+                                             std::int64_t out_row, float factor, int qw, int M) {
+    constexpr int kRowBytes = 128;  // 32 features per pass
+    constexpr int kPasses = kOB;
+    constexpr int kPassesPerHalf = kPasses / 2;  // passes over the first half of the features
+    // The lane's number, counted afresh here: the stage addresses depend on it
+    // only, and kept or computed before the key loop they would hold registers
+    // through it.
+    int none = 0;
+    asm volatile("" : "+v"(none));
+    const int me = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, static_cast<unsigned>(none))));
+    const int my_q = me & 31, my_h = me >> 5;
+    const int c = me & 7, sub = me >> 3;  // read side: chunk c of row sub of each 8-row piece
+#pragma unroll
+    for (int pass = 0; pass < kPasses; ++pass) {
+        // Features 32 pass .. 32 pass + 31: slots
+        // r4 = 2 (pass / kPassesPerHalf) + r of blocks
+        // fb = 2 (pass % kPassesPerHalf) + b hold features
+        // 32 pass + 16 b + 8 r + 4 h (+ 0..3) of row q, i.e. 16-byte
+        // chunk 4 b + 2 r + h of the pass, stored rotated by the row.
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int r4 = 2 * (pass / kPassesPerHalf) + r, fb = 2 * (pass % kPassesPerHalf) + b;
+                const float4v value{st.o[fb][4 * r4], st.o[fb][4 * r4 + 1], st.o[fb][4 * r4 + 2], st.o[fb][4 * r4 + 3]};
+                const int chunk = 4 * b + 2 * r + my_h;
+                *reinterpret_cast<float4v*>(region + my_q * kRowBytes + (((chunk + my_q) & 7) << 4)) = value * factor;
+            }
+        // Piece i: rows 8 i .. 8 i + 7 of the wave, 8 lanes per row. Every
+        // read is issued before any store (the reads stay in the wave's
+        // region; only the stores depend on the row).
+        float4v piece[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int local = 8 * i + sub;
+            piece[i] = *reinterpret_cast<const float4v*>(region + local * kRowBytes + (((c + local) & 7) << 4));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(piece[i]));  // keep the reads here
+        float* const first = out + static_cast<std::int64_t>(qw + sub) * out_row + 32 * pass + 4 * c;
+        const std::int64_t piece_step = 8 * out_row;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (qw + 8 * i + sub < M)
+                __builtin_nontemporal_store(piece[i], reinterpret_cast<float4v*>(first + i * piece_step));
+    }
+}
+
+// A wave's 32 query rows in registers. qf: B operand of the 32x32x16 QK^T
+// MFMA, lane (q, h) holding features 16c + 8h .. 16c + 8h + 7 of its row for
+// chunk c. With INT8 operands also q8f, the B operand of the INT8 MFMA (lane
+// (q, h): features 32m + 16h .. 32m + 16h + 15 for chunk m), and q_scale:
+// quantized here (p.fuse_q_quant) or read from Q8. `group_bits` (shared, one
+// entry per wave of the workgroup, `waves` of them): the maxima of the waves;
+// those of this wave's Q block start at entry `block_first`. Every wave of the
+// workgroup calls it. writer: this workgroup writes Q8 / q_scales where asked.
+template <int DC, int kPiece>
+__device__ __forceinline__ void prepare_q(const AttnParams& p, std::int64_t head, int qblock, int row, int lane,
+                                          unsigned* group_bits, int waves, int wave, int block_first, bool writer,
+                                          half8 (&qf)[2 * DC], int4v (&q8f)[2 * Layout<DC>::kD8C], float& q_scale) {
+    using L = Layout<DC>;
+    constexpr int kQC = 2 * DC;
+    constexpr int kQ8C = 2 * L::kD8C;
+    constexpr bool kVector = kPiece >= 8;
+    const int M = p.M, d = p.d;
+    const int h = lane >> 5;
+    const std::uint16_t* Qh = p.Q + head * p.q_stride;
+    {
+#pragma unroll
+        for (int c = 0; c < kQC; ++c) {
+            const int feature = 16 * c + 8 * h;
+            if constexpr (kVector) {
+                qf[c] = (row < M && feature < d)
+                    ? *reinterpret_cast<const half8*>(Qh + static_cast<std::int64_t>(row) * p.q_row + feature)
+                    : half8{};
+            } else if constexpr (kPiece == 4) {
+                uint4v words{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    if (row < M && feature + 2 * w < d)
+                        words[w] = *reinterpret_cast<const std::uint32_t*>(Qh + static_cast<std::int64_t>(row) * p.q_row + feature + 2 * w);
+                qf[c] = __builtin_bit_cast(half8, words);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    qf[c][e] = (row < M && feature + e < d)
+                        ? __builtin_bit_cast(_Float16, Qh[static_cast<std::int64_t>(row) * p.q_row + feature + e])
+                        : static_cast<_Float16>(0.0f);
+            }
+        }
+    }
+
+    if (p.int8_operands) {
+        if (p.fuse_q_quant) {
+            // Four waves' rows are exactly one 128-row Q block. Its
+            // maximum |x| as fp16 bit patterns: unsigned order is float order
+            // for them, NaN patterns (> 0x7c00) sorting above +inf.
+            unsigned top = 0;
+#pragma unroll
+            for (int c = 0; c < kQC; ++c) {
+                const uint4v words = __builtin_bit_cast(uint4v, qf[c]);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) top = max_u16x2(top, words[w] & 0x7fff7fffu);
+            }
+            unsigned bits = wave_max_bits(max(top & 0xffffu, top >> 16));
+            if (lane == 0) group_bits[wave] = bits;
+            __syncthreads();
+            const unsigned* const block_bits = group_bits + block_first;
+            bits = max(max(block_bits[0], block_bits[1]), max(block_bits[2], block_bits[3]));
+            unsigned any = bits;
+            if (waves > 4)
+                for (int w = 0; w < waves; ++w) any = max(any, group_bits[w]);
+            if (any > 0x7c00u) {
+                // A NaN in the workgroup: the maximum skips NaNs, as fmaxf does.
+                unsigned clean = 0;
+#pragma unroll
+                for (int c = 0; c < kQC; ++c)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        // The element is copied out first: __builtin_bit_cast
+                        // applied to a vector element expression reads
+                        // element 0 under this compiler.
+                        const _Float16 x = qf[c][e];
+                        const unsigned hb = __builtin_bit_cast(std::uint16_t, x) & 0x7fffu;
+                        clean = hb <= 0x7c00u ? max(clean, hb) : clean;
+                    }
+                clean = wave_max_bits(clean);
+                __syncthreads();
+                if (lane == 0) group_bits[wave] = clean;
+                __syncthreads();
+                bits = max(max(block_bits[0], block_bits[1]), max(block_bits[2], block_bits[3]));
+            }
+            const float scale = block_scale(half_bits_to_float(static_cast<std::uint16_t>(bits)));
+            const float recip = 1.0f / scale;
+            const _Float16 stored = static_cast<_Float16>(scale);
+            q_scale = static_cast<float>(stored);
+            if (writer && p.q_scales_out && wave == block_first && lane == 0)
+                p.q_scales_out[head * p.q_blocks + qblock] = __builtin_bit_cast(std::uint16_t, stored);
+            {
+                // Bytes of fp16 chunk c (features 16c + 8h .. + 7 of the row).
+                uint2v packed[L::kDP8 / 16];
+#pragma unroll
+                for (int c = 0; c < L::kDP8 / 16; ++c) {
+                    packed[c] = uint2v{0u, 0u};
+                    if (c < kQC && scale > 0.0f) {
+                        const uint4v words = __builtin_bit_cast(uint4v, qf[c < kQC ? c : 0]);
+                        int v[8];
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            v[2 * w] = quantize_half<0>(words[w], scale, recip);
+                            v[2 * w + 1] = quantize_half<1>(words[w], scale, recip);
+                        }
+                        packed[c][0] = pack_bytes(v[0], v[1], v[2], v[3]);
+                        packed[c][1] = pack_bytes(v[4], v[5], v[6], v[7]);
+                    }
+                    const int feature = 16 * c + 8 * h;
+                    if (p.q8_out && writer && row < M && feature < d) {
+                        std::int8_t* dst = p.q8_out + head * static_cast<std::int64_t>(M) * d +
+                                           static_cast<std::int64_t>(row) * d + feature;
+                        if constexpr (kVector) {
+                            *reinterpret_cast<uint2v*>(dst) = packed[c];
+                        } else {
+                            for (int e = 0; e < 8 && feature + e < d; ++e)
+                                dst[e] = static_cast<std::int8_t>(packed[c][e / 4] >> (8 * (e % 4)));
+                        }
+                    }
+                }
+                // INT8 chunk m = fp16 chunks 2m (features 32m .. 32m + 15)
+                // and 2m + 1 (32m + 16 .. 32m + 31). Lanes h = 0 keep their
+                // bytes of chunk 2m and take lane (q, 1)'s; lanes h = 1 keep
+                // their bytes of chunk 2m + 1 and take lane (q, 0)'s: one
+                // v_permlane32_swap per dword.
+#pragma unroll
+                for (int m = 0; m < kQ8C; ++m) {
+                    const uint2v keep = h ? packed[2 * m + 1] : packed[2 * m];
+                    const uint2v send = h ? packed[2 * m] : packed[2 * m + 1];
+                    std::uint32_t got[2];
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) {
+                        const std::uint32_t word = send[k];  // copied out before the bit cast, see above
+                        float a = __builtin_bit_cast(float, word), b = a;
+                        permlane32_swap(a, b);  // a: lane (q, 0)'s dword, b: lane (q, 1)'s
+                        got[k] = __builtin_bit_cast(std::uint32_t, h ? a : b);
+                    }
+                    q8f[m] = h ? int4v{static_cast<int>(got[0]), static_cast<int>(got[1]), static_cast<int>(keep[0]),
+                                       static_cast<int>(keep[1])}
+                               : int4v{static_cast<int>(keep[0]), static_cast<int>(keep[1]), static_cast<int>(got[0]),
+                                       static_cast<int>(got[1])};
+                }
+            }
+        } else {
+            // Q8 rows already come in the operand layout: 16 bytes per lane
+            // and chunk, read straight into q8f.
+            q_scale = half_bits_to_float(p.q_scales[head * p.q_blocks + qblock]);
+            const std::int8_t* Q8h = p.Q8 + head * static_cast<std::int64_t>(M) * d;
+#pragma unroll
+            for (int m = 0; m < kQ8C; ++m) {
+                const int feature = 32 * m + 16 * h;
+                int4v chunk;
+                if constexpr (kPiece == 16) {
+                    chunk = (row < M && feature < d)
+                        ? *reinterpret_cast<const int4v*>(Q8h + static_cast<std::int64_t>(row) * d + feature)
+                        : int4v{0, 0, 0, 0};
+                } else if constexpr (kPiece != 0) {
+                    chunk = int4v{0, 0, 0, 0};
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        if (row < M && feature + 4 * w < d)
+                            chunk[w] = *reinterpret_cast<const int*>(Q8h + static_cast<std::int64_t>(row) * d + feature + 4 * w);
+                } else {
+                    unsigned char bytes[16];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        bytes[e] = (row < M && feature + e < d)
+                            ? static_cast<unsigned char>(Q8h[static_cast<std::int64_t>(row) * d + feature + e])
+                            : 0;
+                    chunk = __builtin_bit_cast(int4v, bytes);
+                }
+                q8f[m] = chunk;
+            }
+        }
+    }
 }
 
 // kPiece: what rows allow (access_piece). 16: tiles move by LDS DMA in 16-byte
@@ -319,175 +568,16 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         }
     }
 
-    const std::uint16_t* Qh = p.Q + head * p.q_stride;
     const std::uint16_t* Kh = p.K + head * p.k_stride;
     const std::uint16_t* Vh = p.V + head * p.v_stride;
     const std::int8_t* K8h = p.K8 + head * static_cast<std::int64_t>(N) * d;
     unsigned char* const Oh = static_cast<unsigned char*>(p.O) + head * p.o_stride * (p.o_dtype == TILEMIX_DTYPE_F32 ? 4 : 2);
 
     // ---------------------------------------------------------------- Q
-    // B operand of the 32x32x16 QK^T MFMA: lane (q, h) holds features
-    // 16c + 8h .. 16c + 8h + 7 of its row for chunk c.
     half8 qf[kQC];
-    {
-        const int row = qw + q;
-#pragma unroll
-        for (int c = 0; c < kQC; ++c) {
-            const int feature = 16 * c + 8 * h;
-            if constexpr (kVector) {
-                qf[c] = (row < M && feature < d)
-                    ? *reinterpret_cast<const half8*>(Qh + static_cast<std::int64_t>(row) * p.q_row + feature)
-                    : half8{};
-            } else if constexpr (kPiece == 4) {
-                uint4v words{0u, 0u, 0u, 0u};
-#pragma unroll
-                for (int w = 0; w < 4; ++w)
-                    if (row < M && feature + 2 * w < d)
-                        words[w] = *reinterpret_cast<const std::uint32_t*>(Qh + static_cast<std::int64_t>(row) * p.q_row + feature + 2 * w);
-                qf[c] = __builtin_bit_cast(half8, words);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    qf[c][e] = (row < M && feature + e < d)
-                        ? __builtin_bit_cast(_Float16, Qh[static_cast<std::int64_t>(row) * p.q_row + feature + e])
-                        : static_cast<_Float16>(0.0f);
-            }
-        }
-    }
-
-    // The wave's quantized Q rows (B operand of the INT8 MFMA), kept in
-    // registers: lane (q, h) holds features 32m + 16h .. 32m + 16h + 15 of
-    // its row for chunk m.
     int4v q8f[kQ8C];
     float q_scale = 0.0f;
-    if (p.int8_operands) {
-        if (p.fuse_q_quant) {
-            // The workgroup's rows are exactly one 128-row Q block. Its
-            // maximum |x| as fp16 bit patterns: unsigned order is float order
-            // for them, NaN patterns (> 0x7c00) sorting above +inf.
-            unsigned top = 0;
-#pragma unroll
-            for (int c = 0; c < kQC; ++c) {
-                const uint4v words = __builtin_bit_cast(uint4v, qf[c]);
-#pragma unroll
-                for (int w = 0; w < 4; ++w) top = max_u16x2(top, words[w] & 0x7fff7fffu);
-            }
-            unsigned bits = wave_max_bits(max(top & 0xffffu, top >> 16));
-            if (lane == 0) group_bits[wave] = bits;
-            __syncthreads();
-            bits = max(max(group_bits[0], group_bits[1]), max(group_bits[2], group_bits[3]));
-            if (bits > 0x7c00u) {
-                // A NaN in the block: the maximum skips NaNs, as fmaxf does.
-                unsigned clean = 0;
-#pragma unroll
-                for (int c = 0; c < kQC; ++c)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        // The element is copied out first: __builtin_bit_cast
-                        // applied to a vector element expression reads
-                        // element 0 under this compiler.
-                        const _Float16 x = qf[c][e];
-                        const unsigned hb = __builtin_bit_cast(std::uint16_t, x) & 0x7fffu;
-                        clean = hb <= 0x7c00u ? max(clean, hb) : clean;
-                    }
-                clean = wave_max_bits(clean);
-                __syncthreads();
-                if (lane == 0) group_bits[wave] = clean;
-                __syncthreads();
-                bits = max(max(group_bits[0], group_bits[1]), max(group_bits[2], group_bits[3]));
-            }
-            const float scale = block_scale(half_bits_to_float(static_cast<std::uint16_t>(bits)));
-            const float recip = 1.0f / scale;
-            const _Float16 stored = static_cast<_Float16>(scale);
-            q_scale = static_cast<float>(stored);
-            if (tid == 0 && p.q_scales_out && split == 0)
-                p.q_scales_out[head * p.q_blocks + qblock] = __builtin_bit_cast(std::uint16_t, stored);
-            {
-                const int row = qw + q;
-                // Bytes of fp16 chunk c (features 16c + 8h .. + 7 of the row).
-                uint2v packed[L::kDP8 / 16];
-#pragma unroll
-                for (int c = 0; c < L::kDP8 / 16; ++c) {
-                    packed[c] = uint2v{0u, 0u};
-                    if (c < kQC && scale > 0.0f) {
-                        const uint4v words = __builtin_bit_cast(uint4v, qf[c < kQC ? c : 0]);
-                        int v[8];
-#pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            v[2 * w] = quantize_half<0>(words[w], scale, recip);
-                            v[2 * w + 1] = quantize_half<1>(words[w], scale, recip);
-                        }
-                        packed[c][0] = pack_bytes(v[0], v[1], v[2], v[3]);
-                        packed[c][1] = pack_bytes(v[4], v[5], v[6], v[7]);
-                    }
-                    const int feature = 16 * c + 8 * h;
-                    if (p.q8_out && split == 0 && row < M && feature < d) {
-                        std::int8_t* dst = p.q8_out + head * static_cast<std::int64_t>(M) * d +
-                                           static_cast<std::int64_t>(row) * d + feature;
-                        if constexpr (kVector) {
-                            *reinterpret_cast<uint2v*>(dst) = packed[c];
-                        } else {
-                            for (int e = 0; e < 8 && feature + e < d; ++e)
-                                dst[e] = static_cast<std::int8_t>(packed[c][e / 4] >> (8 * (e % 4)));
-                        }
-                    }
-                }
-                // INT8 chunk m = fp16 chunks 2m (features 32m .. 32m + 15)
-                // and 2m + 1 (32m + 16 .. 32m + 31). Lanes h = 0 keep their
-                // bytes of chunk 2m and take lane (q, 1)'s; lanes h = 1 keep
-                // their bytes of chunk 2m + 1 and take lane (q, 0)'s: one
-                // v_permlane32_swap per dword.
-#pragma unroll
-                for (int m = 0; m < kQ8C; ++m) {
-                    const uint2v keep = h ? packed[2 * m + 1] : packed[2 * m];
-                    const uint2v send = h ? packed[2 * m] : packed[2 * m + 1];
-                    std::uint32_t got[2];
-#pragma unroll
-                    for (int k = 0; k < 2; ++k) {
-                        const std::uint32_t word = send[k];  // copied out before the bit cast, see above
-                        float a = __builtin_bit_cast(float, word), b = a;
-                        permlane32_swap(a, b);  // a: lane (q, 0)'s dword, b: lane (q, 1)'s
-                        got[k] = __builtin_bit_cast(std::uint32_t, h ? a : b);
-                    }
-                    q8f[m] = h ? int4v{static_cast<int>(got[0]), static_cast<int>(got[1]), static_cast<int>(keep[0]),
-                                       static_cast<int>(keep[1])}
-                               : int4v{static_cast<int>(keep[0]), static_cast<int>(keep[1]), static_cast<int>(got[0]),
-                                       static_cast<int>(got[1])};
-                }
-            }
-        } else {
-            // Q8 rows already come in the operand layout: 16 bytes per lane
-            // and chunk, read straight into q8f.
-            q_scale = half_bits_to_float(p.q_scales[head * p.q_blocks + qblock]);
-            const std::int8_t* Q8h = p.Q8 + head * static_cast<std::int64_t>(M) * d;
-            const int row = qw + q;
-#pragma unroll
-            for (int m = 0; m < kQ8C; ++m) {
-                const int feature = 32 * m + 16 * h;
-                int4v chunk;
-                if constexpr (kPiece == 16) {
-                    chunk = (row < M && feature < d)
-                        ? *reinterpret_cast<const int4v*>(Q8h + static_cast<std::int64_t>(row) * d + feature)
-                        : int4v{0, 0, 0, 0};
-                } else if constexpr (kPiece != 0) {
-                    chunk = int4v{0, 0, 0, 0};
-#pragma unroll
-                    for (int w = 0; w < 4; ++w)
-                        if (row < M && feature + 4 * w < d)
-                            chunk[w] = *reinterpret_cast<const int*>(Q8h + static_cast<std::int64_t>(row) * d + feature + 4 * w);
-                } else {
-                    unsigned char bytes[16];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        bytes[e] = (row < M && feature + e < d)
-                            ? static_cast<unsigned char>(Q8h[static_cast<std::int64_t>(row) * d + feature + e])
-                            : 0;
-                    chunk = __builtin_bit_cast(int4v, bytes);
-                }
-                q8f[m] = chunk;
-            }
-        }
-    }
+    prepare_q<DC, kPiece>(p, head, qblock, qw + q, lane, group_bits, kWavesPerGroup, wave, 0, split == 0, qf, q8f, q_scale);
 
     // Key tiles are visited first to last, or last to first in a reversed
     // round (AttnParams::reverse_slots; the online softmax takes the tiles in
@@ -960,79 +1050,18 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         }
     }
 
-    // fp32 rows of 128 or 64 features (O, or a split's partial rows) leave
-    // the variants without dot export through LDS. From registers, each
-    // store instruction writes 16 bytes to each of 32 rows, i.e. 32 partial
-    // cache lines, and those lines, held in the XCD's L2 until written back,
-    // evict K / V tiles. Staged, each store writes 8 rows x 128 bytes (full
-    // cache lines) with a non-temporal hint, so the rows bypass the L2. The stage buffers
-    // are the K tile buffer (both 4 KiB regions of it at d = 64, all four
-    // at d = 128) and at d = 64 the V buffer the last tile did not use:
-    // every wave has passed the last tile's second barrier, so no wave
-    // reads them any more and no load targets them. Each wave stages its
-    // 32 rows in kDP / 32 passes of 32 features through a 4 KiB region.
-    // out / out_row: the head's first row and the distance between rows, in
-    // floats; every value is multiplied by factor.
+    // Staged stores (store_staged): the regions are the K tile buffer (both 4
+    // KiB regions of it at d = 64, all four at d = 128) and at d = 64 the V
+    // buffer the last tile did not use: every wave has passed the last tile's
+    // second barrier, so no wave reads them any more and no load targets them.
     constexpr bool kStaged = kPiece == 16 && !kDots && (kDP == 128 || kDP == 64);
-    auto store_staged = [&](float* out, std::int64_t out_row, float factor) {
-        if constexpr (kStaged) {
-            constexpr int kRowBytes = 128;           // 32 features per pass
-            constexpr int kRegion = 32 * kRowBytes;  // 4 KiB per wave
-            constexpr int kPasses = kDP / 32;
-            constexpr int kPassesPerHalf = kPasses / 2;  // passes over features [0, kDP / 2)
-            unsigned char* region;
-            if constexpr (kDP == 128) {
-                static_assert(L::kKBytes >= kWavesPerGroup * kRegion, "stage regions fit the K buffer");
-                region = lds_k + wave * kRegion;
-            } else {
-                static_assert(L::kKBytes >= 2 * kRegion && L::kVBytes >= 2 * kRegion, "stage regions fit K and V");
-                region = wave < 2 ? lds_k + wave * kRegion : lds_v + (v_buffer ? L::kV1Offset : 0) + (wave - 2) * kRegion;
-            }
-            // The lane's position, taken afresh here: the stage addresses
-            // depend on the lane only, and computed before the key loop
-            // they would hold registers through it.
-            int me = lane;
-            asm volatile("" : "+v"(me));
-            const int my_q = me & 31, my_h = me >> 5;
-            const int c = me & 7, sub = me >> 3;  // read side: chunk c of row sub of each 8-row piece
-#pragma unroll
-            for (int pass = 0; pass < kPasses; ++pass) {
-                // Features 32 pass .. 32 pass + 31: slots
-                // r4 = 2 (pass / kPassesPerHalf) + r of blocks
-                // fb = 2 (pass % kPassesPerHalf) + b hold features
-                // 32 pass + 16 b + 8 r + 4 h (+ 0..3) of row q, i.e. 16-byte
-                // chunk 4 b + 2 r + h of the pass, stored rotated by the row.
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int r = 0; r < 2; ++r) {
-                        const int r4 = 2 * (pass / kPassesPerHalf) + r, fb = 2 * (pass % kPassesPerHalf) + b;
-                        const float4v value{st.o[fb][4 * r4], st.o[fb][4 * r4 + 1], st.o[fb][4 * r4 + 2],
-                                            st.o[fb][4 * r4 + 3]};
-                        const int chunk = 4 * b + 2 * r + my_h;
-                        *reinterpret_cast<float4v*>(region + my_q * kRowBytes + (((chunk + my_q) & 7) << 4)) =
-                            value * factor;
-                    }
-                // Piece i: rows 8 i .. 8 i + 7 of the wave, 8 lanes per row.
-                // Every read is issued before any store (the reads stay in
-                // the wave's region; only the stores depend on the row).
-                float4v piece[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int local = 8 * i + sub;
-                    piece[i] = *reinterpret_cast<const float4v*>(region + local * kRowBytes + (((c + local) & 7) << 4));
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(piece[i]));  // keep the reads here
-                float* const first = out + static_cast<std::int64_t>(qw + sub) * out_row + 32 * pass + 4 * c;
-                const std::int64_t piece_step = 8 * out_row;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (qw + 8 * i + sub < M)
-                        __builtin_nontemporal_store(piece[i], reinterpret_cast<float4v*>(first + i * piece_step));
-            }
-        }
-    };
+    unsigned char* stage = lds_k + wave * kStageBytes;
+    if constexpr (kStaged && kDP == 64) {
+        static_assert(L::kKBytes >= 2 * kStageBytes && L::kVBytes >= 2 * kStageBytes, "stage regions fit K and V");
+        if (wave >= 2) stage = lds_v + (v_buffer ? L::kV1Offset : 0) + (wave - 2) * kStageBytes;
+    } else if constexpr (kStaged) {
+        static_assert(L::kKBytes >= kWavesPerGroup * kStageBytes, "stage regions fit the K buffer");
+    }
     // ---------------------------------------------------------- epilogue
     if constexpr (kSplit) {
         // This split's unnormalised rows and their (m, l), for the combine.
@@ -1041,7 +1070,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         const int row = qw + q;
         if constexpr (kStaged) {
             if (d == kDP) {
-                store_staged(p.part_o + part * d, d, 1.0f);
+                store_staged<kOB>(st, stage, p.part_o + part * d, d, 1.0f, qw, M);
                 if (row < M && h == 0) {
                     float* const ml = p.part_ml + 2 * (part + row);
                     ml[0] = st.m;
@@ -1075,7 +1104,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         const int row = qw + q;
         if constexpr (kStaged) {
             if (p.o_dtype == TILEMIX_DTYPE_F32 && d == kDP) {
-                store_staged(reinterpret_cast<float*>(Oh), p.o_row, inverse);
+                store_staged<kOB>(st, stage, reinterpret_cast<float*>(Oh), p.o_row, inverse, qw, M);
                 return;
             }
         }
@@ -1092,6 +1121,488 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                     store_output(Oh, p.o_dtype, row_offset + feature, value * inverse, d - feature, kVector || p.o_vector);
                 }
         }
+    }
+}
+
+// ------------------------------------------------------------- wide kernel
+//
+// The same rows, arithmetic and tile order as attention_kernel, for launches
+// with enough row blocks: one workgroup of eight waves per CU owns 256 query
+// rows (two Q quantization blocks), so each K / K8 / V tile is loaded into LDS
+// once for 256 rows instead of 128, and its two halves (waves 0-3 and 4-7, one
+// wave of each on every SIMD) run half a tile apart. A tile is two slots
+// between barriers of the whole workgroup:
+//   matrix slot  P.V of the previous tile, then this tile's scores;
+//   vector slot  routes, masks and softmax of this tile.
+// The second half enters one barrier later, so in every slot one wave of each
+// SIMD has the matrix core while the other runs exponentials. Tile buffers are
+// all double: K (i + 1) and V (i) of walk position i are fetched from the slot
+// in which the first half starts position i (the slot before, the second half
+// finished the tiles that were there) and waited for two slots later:
+//   slot         2i              2i + 1
+//   first half   P.V i-1, QK i   softmax i
+//   second half  softmax i-1     P.V i-1, QK i
+//   loads        issue K i+1, V i; all waves wait for them at the end of 2i+1
+// Everything a wave has to know of a tile is decided once, before the walk:
+// the visited tiles of the workgroup, in walking order, with the wave's cells
+// as one word each (Entry). Tile offsets go into the lanes' offsets, which the
+// buffer range check covers, so a tail tile is loaded like any other, and the
+// walk is unrolled twice so that buffers are constants: a tile's scalar work is
+// a few instructions. (With the routes decoded in the walk, tail tiles through
+// views of their own and buffers in variables, the slots' control alone took
+// half of the kernel's time.)
+// What bounds it, at 128 features, dense (32 heads x 8192: 1033 us, 1.06
+// PFLOP/s; 1064 us with attention_kernel): about 1800 cycles a slot at 1.79 GHz
+// under the power limit. The matrix slot alone takes 1540 (1024 of them MFMAs;
+// the LDS reads of V's transposed fragments, at half the rate of K's, take
+// longer than the P.V MFMAs they feed), the vector slot alone 1500 (32
+// exponentials at 16 cycles, 110 other instructions). Interleaving P.V with the
+// scores MFMA by MFMA spilled 160 registers at 128 features and was 3 % slower
+// at 64; three tile buffers of each were no faster.
+constexpr int kWideThreads = 512;
+#define TILEMIX_INLINE __attribute__((always_inline))  // lambdas the walk uses twice
+constexpr int kWideWaves = kWideThreads / kWave;
+constexpr int kWideRows = 256;
+constexpr int kWideMaxTiles = 1024;  // key tiles that the table holds
+
+// A wave's view of one visited tile: cell bits (2 r + key half) in INT8 and
+// SKIP, what any wave of the workgroup needs of it, how this wave scores it.
+struct Entry {
+    static constexpr unsigned kInt8 = 0xfu, kSkipShift = 4;
+    static constexpr unsigned kNeeds16 = 1u << 8, kNeeds8 = 1u << 9, kVisited = 1u << 10;
+    static constexpr unsigned kModeShift = 11;  // 2 bits
+    static constexpr unsigned kFp16 = 0, kAllInt8 = 1, kMixed = 2, kIdle = 3;
+    static constexpr unsigned kMasked = 1u << 13;  // holds keys that some row of the wave does not see
+    static constexpr unsigned kTileShift = 16;
+    static constexpr unsigned kEnd = kIdle << kModeShift;
+};
+
+template <int DC>
+__global__ __launch_bounds__(kWideThreads, 1) void attention_wide_kernel(const AttnParams p) {
+    using L = Layout<DC>;
+    constexpr int kDP = L::kDP;
+    constexpr int kOB = DC;
+    constexpr int kQC = kDP / 16;
+    constexpr int kQ8C = L::kDP8 / 32;
+    static_assert(L::kRotate && L::kRotate8, "wide kernel: rotated rows");
+    // K0 K1 | K8_0 K8_1 | V0 V1
+    constexpr int kK8Base = 2 * L::kKBytes, kVBase = kK8Base + 2 * L::kK8Bytes;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kVBase + 2 * L::kVBytes];
+    __shared__ unsigned group_bits[kWideWaves];
+    __shared__ unsigned entries[kWideWaves][kWideMaxTiles];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool second = wave >= kWideWaves / 2;
+    const int i = lane & 15;
+    const int q = lane & 31;
+    const int h = lane >> 5;
+    const int blocks = (p.q_blocks + 1) / 2;
+    int head32, block;
+    map_block(blockIdx.x, p.heads, blocks, p.causal != 0, head32, block);
+    const std::int64_t head = head32;
+    const int q0 = block * kWideRows;
+    const int qw = q0 + wave * kRowsPerWave;
+    const int M = p.M, N = p.N, d = p.d;
+
+    // ------------------------------------------------------ route table
+    int tiles = (N - 1) / kTileKeys + 1;
+    if (p.causal) tiles = min(tiles, (q0 + kWideRows - 1) / kTileKeys + 1);
+    const bool reversed = reversed_round(blockIdx.x, p.reverse_slots);
+    {
+        const int qt = qw / 16;
+        const std::int64_t words = head * p.words_per_head + static_cast<std::int64_t>(qt) * p.words_per_row;
+        for (int x = lane; x < tiles; x += kWave) {
+            const int tile = reversed ? tiles - 1 - x : x;
+            unsigned int8 = 0, skip = 0;
+#pragma unroll
+            for (int cell = 0; cell < 4; ++cell) {
+                const int r = cell >> 1, kt = 2 * tile + (cell & 1);
+                bool is_skip = qt + r >= p.q_tiles16 || kt >= p.key_tiles32, is_int8 = false;
+                if (!is_skip && (p.route_words || p.skip_words)) {
+                    const unsigned group = p.group_shift >= 0 ? static_cast<unsigned>(kt) >> p.group_shift
+                                                              : static_cast<unsigned>(kt) / static_cast<unsigned>(p.key_tiles_per_group);
+                    const std::int64_t word = words + r * p.words_per_row + (group >> 6);
+                    const unsigned bit = group & 63u;
+                    is_skip = p.skip_words && ((p.skip_words[word] >> bit) & 1u);
+                    is_int8 = !is_skip && p.route_words && ((p.route_words[word] >> bit) & 1u);
+                }
+                int8 |= static_cast<unsigned>(is_int8) << cell;
+                skip |= static_cast<unsigned>(is_skip) << cell;
+            }
+            // No row of the wave, or none that sees a key of the tile.
+            const int k0 = tile * kTileKeys;
+            if (qw >= M || (p.causal && k0 > qw + kRowsPerWave - 1)) {
+                int8 = 0;
+                skip = 0xfu;
+            }
+            const bool masked = k0 + kTileKeys > N || (p.causal && k0 + kTileKeys - 1 > qw);
+            const unsigned mode = skip == 0xfu ? Entry::kIdle
+                                  : skip != 0  ? Entry::kMixed
+                                  : int8 == 0  ? Entry::kFp16
+                                               : (int8 == 0xfu ? Entry::kAllInt8 : Entry::kMixed);
+            entries[wave][x] = int8 | (skip << Entry::kSkipShift) | (mode << Entry::kModeShift) |
+                               (masked ? Entry::kMasked : 0u) | (static_cast<unsigned>(tile) << Entry::kTileShift);
+        }
+    }
+
+    half8 qf[kQC];
+    int4v q8f[kQ8C];
+    float q_scale = 0.0f;
+    const int qblock = min(2 * block + (second ? 1 : 0), p.q_blocks - 1);
+    prepare_q<DC, 16>(p, head, qblock, qw + q, lane, group_bits, kWideWaves, wave, second ? kWideWaves / 2 : 0,
+                      2 * block + (second ? 1 : 0) < p.q_blocks, qf, q8f, q_scale);
+
+    // What any wave needs of a tile, and the visited tiles moved to the front
+    // (in place: a wave's entry moves to its own or an earlier place; what the
+    // other waves' words say is read before any word moves).
+    int count = 0;
+    for (int first = 0; first < tiles; first += kWave) {
+        __syncthreads();
+        const int x = first + lane;
+        unsigned mine = Entry::kEnd, needs = 0;
+        if (x < tiles) {
+            mine = entries[wave][x];
+#pragma unroll
+            for (int w = 0; w < kWideWaves; ++w) {
+                const unsigned word = entries[w][x], int8 = word & Entry::kInt8, skip = (word >> Entry::kSkipShift) & 0xfu;
+                needs |= (skip != 0xfu ? Entry::kVisited : 0u) | (((~int8 & ~skip) & 0xfu) ? Entry::kNeeds16 : 0u) |
+                         (int8 ? Entry::kNeeds8 : 0u);
+            }
+        }
+        const std::uint64_t visited = __ballot(needs != 0);
+        __syncthreads();
+        if (needs)
+            entries[wave][count + __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(visited >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(visited), 0u))] =
+                mine | needs;
+        count += __popcll(visited);
+    }
+    // Lane l of the window holds the entry at position window + l (kEnd past
+    // the last) and its K block's scale.
+    int window = 0;
+    unsigned window_entry;
+    float window_scale = 0.0f;
+    auto load_window = [&]() TILEMIX_INLINE {
+        const int at = window + lane;
+        window_entry = at < count ? entries[wave][at] : Entry::kEnd;
+        if (p.int8_operands && at < count)
+            window_scale = half_bits_to_float(p.k_scales[head * p.k_blocks + (window_entry >> Entry::kTileShift)]);
+    };
+    struct Position {
+        unsigned entry;
+        float k_scale;
+    };
+    auto position = [&](int x) TILEMIX_INLINE {
+        if (x - window >= kWave) {
+            window += kWave;
+            load_window();
+        }
+        return Position{static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(window_entry), x - window)),
+                        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, window_scale), x - window))};
+    };
+
+    // ------------------------------------------------------ tile movement
+    const int4v rsrc_k = make_rsrc(p.K + head * p.k_stride, static_cast<int>((static_cast<std::int64_t>(N - 1) * p.k_row + d) * 2));
+    const int4v rsrc_v = make_rsrc(p.V + head * p.v_stride, static_cast<int>((static_cast<std::int64_t>(N - 1) * p.v_row + d) * 2));
+    const int4v rsrc_k8 = make_rsrc(p.K8 + (p.int8_operands ? head * static_cast<std::int64_t>(N) * d : 0),
+                                    static_cast<int>(p.int8_operands ? static_cast<std::int64_t>(N) * d : 0));
+    const int k_tile_bytes = static_cast<int>(p.k_row * 2 * kTileKeys), v_tile_bytes = static_cast<int>(p.v_row * 2 * kTileKeys);
+    const int k8_tile_bytes = d * kTileKeys;
+    constexpr int kKSlots = L::kKLoads / kWideWaves, kVSlots = L::kVLoads / kWideWaves;
+    static_assert(L::kKLoads % kWideWaves == 0 && L::kVLoads % kWideWaves == 0 && L::kK8Loads <= kWideWaves,
+                  "K and V split evenly over the waves, K8 is one piece at most");
+    int off_k[kKSlots], off_v[kVSlots];
+#pragma unroll
+    for (int t = 0; t < kKSlots; ++t)
+        off_k[t] = L::template kv_lane_offset<true>(wave + kWideWaves * t, lane, L::kKStride, 2 * d, static_cast<int>(p.k_row * 2));
+#pragma unroll
+    for (int t = 0; t < kVSlots; ++t)
+        off_v[t] = L::template kv_lane_offset<false>(wave + kWideWaves * t, lane, L::kVStride, 2 * d, static_cast<int>(p.v_row * 2));
+    const bool k8_mover = wave < L::kK8Loads;
+    const int off_k8 = k8_mover ? L::k8_lane_offset(wave, lane, d) : kOutOfRange;
+    // This wave's first piece of a tile, from the start of a buffer.
+    const unsigned lds_wave = lds_address_of(smem) + 1024 * wave;
+    auto issue_k = [&](unsigned entry, auto buffer) TILEMIX_INLINE {
+        constexpr int b = decltype(buffer)::value;
+        const int tile = static_cast<int>(entry >> Entry::kTileShift);
+        if (entry & Entry::kNeeds16) load_slots_at<b * L::kKBytes, 0, kKSlots>(rsrc_k, lds_wave, off_k, tile * k_tile_bytes);
+        if ((entry & Entry::kNeeds8) && k8_mover)
+            load_to_lds_at<kK8Base + b * L::kK8Bytes>(rsrc_k8, lds_wave, off_k8 + tile * k8_tile_bytes, 0);
+    };
+    auto issue_v = [&](unsigned entry, auto buffer) TILEMIX_INLINE {
+        constexpr int b = decltype(buffer)::value;
+        if (entry & Entry::kVisited)
+            load_slots_at<kVBase + b * L::kVBytes, 0, kVSlots>(rsrc_v, lds_wave, off_v,
+                                                                static_cast<int>(entry >> Entry::kTileShift) * v_tile_bytes);
+    };
+
+    int k_lane[kQC], v_lane[kOB], k8_lane[kQ8C];
+#pragma unroll
+    for (int m = 0; m < kQ8C; ++m) k8_lane[m] = kK8Base + L::k8_at(q, 32 * m + 16 * h);
+#pragma unroll
+    for (int c = 0; c < kQC; ++c) k_lane[c] = L::k_at(q, 32 * c + 16 * h);
+#pragma unroll
+    for (int fb = 0; fb < kOB; ++fb)
+        v_lane[fb] = kVBase + L::v_at(4 * h + (i >> 2), 2 * (16 * fb + (kDP / 2) * ((lane >> 4) & 1) + 4 * (i & 3)));
+
+    RowState<kOB> st;
+#pragma unroll
+    for (int fb = 0; fb < kOB; ++fb) st.o[fb] = float16v{};
+    st.lsum = 0.0f;
+    st.m = -INFINITY;
+    const unsigned explicit_scores = p.score_scale >= 0.0f ? 0u : 1u;
+    float16v s[2];      // scores, or (INT8 tiles) the bits of their int32 dots, matrix slot -> vector slot
+    half8 ph[4], unused[4];  // probabilities, vector slot -> next matrix slot
+    bool pv_pending = false;
+
+    // Exact int32 dots / fp16 scores of both key blocks.
+    auto fp16_scores = [&](auto buffer, float16v (&x)[2]) TILEMIX_INLINE {
+        constexpr int kAt = decltype(buffer)::value * L::kKBytes;
+        x[0] = float16v{};
+        x[1] = float16v{};
+        half8 kf[3][2];
+        auto load_c = [&](int cc, half8 (&dst)[2]) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                dst[kb] = *reinterpret_cast<const half8*>(smem + kAt + 32 * L::kKStride * kb + k_lane[cc]);
+        };
+        load_c(0, kf[0]);
+        load_c(1, kf[1]);
+#pragma unroll
+        for (int cc = 0; cc < kQC; ++cc) {
+            if (cc + 2 < kQC) load_c(cc + 2, kf[(cc + 2) % 3]);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                x[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[cc % 3][kb], qf[cc], x[kb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto int8_scores = [&](auto buffer, int16v (&acc)[2]) TILEMIX_INLINE {
+        constexpr int kAt = decltype(buffer)::value * L::kK8Bytes;
+        acc[0] = int16v{};
+        acc[1] = int16v{};
+        int4v kf8[2][2];
+        auto load_m = [&](int m, int4v (&dst)[2]) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                dst[kb] = *reinterpret_cast<const int4v*>(smem + kAt + 32 * L::kK8Stride * kb + k8_lane[m]);
+        };
+        load_m(0, kf8[0]);
+#pragma unroll
+        for (int m = 0; m < kQ8C; ++m) {
+            if (m + 1 < kQ8C) load_m(m + 1, kf8[(m + 1) & 1]);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                acc[kb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf8[m & 1][kb], q8f[m], acc[kb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto k_factor_of = [&](const Position& at) TILEMIX_INLINE { return ((q_scale * at.k_scale) * p.score_scale) * kLog2e; };
+
+    // ------------------------------------------------------- matrix slot
+    // P.V of the tile before, then the scores of position `at`; the read
+    // offsets flip to the other buffers with each.
+    auto probabilities_times_values = [&](auto buffer) TILEMIX_INLINE {
+        constexpr int kAt = decltype(buffer)::value * L::kVBytes;
+        if (!pv_pending) return;
+        auto v_frag = [&](int t) TILEMIX_INLINE {
+            const unsigned char* v_lo = smem + kAt + 16 * L::kVStride * (t / kOB) + v_lane[t % kOB];
+            return concat(read_tr16(v_lo), read_tr16(v_lo + 8 * L::kVStride));
+        };
+        constexpr int kSteps = 4 * kOB;
+        constexpr int kAhead = 3;
+        half8 vf[kAhead + 1];
+#pragma unroll
+        for (int t = 0; t < kAhead; ++t)
+            if (t < kSteps) vf[t] = v_frag(t);
+#pragma unroll
+        for (int t = 0; t < kSteps; ++t) {
+            if (t + kAhead < kSteps) vf[(t + kAhead) % (kAhead + 1)] = v_frag(t + kAhead);
+            const int ks = t / kOB, fb = t % kOB;
+            st.o[fb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[t % (kAhead + 1)], ph[ks], st.o[fb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto scores = [&](const Position& at, auto buffer) TILEMIX_INLINE {
+        // The scores of the position before end here, on every path: on that of
+        // an idle wave they would otherwise stay in registers through P.V.
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) asm volatile("" : "=v"(s[kb]));
+        const unsigned mode = (at.entry >> Entry::kModeShift) & 3u;
+        if (mode == Entry::kFp16) {
+            fp16_scores(buffer, s);
+        } else if (mode == Entry::kAllInt8) {
+            int16v acc[2];
+            int8_scores(buffer, acc);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) s[kb] = __builtin_bit_cast(float16v, acc[kb]);
+        } else if (mode == Entry::kMixed) {
+            const unsigned int8 = at.entry & Entry::kInt8, skip = (at.entry >> Entry::kSkipShift) & 0xfu;
+            // Both kinds where present, explicitly scaled, then
+            // selected per lane (cell bit 2 (q / 16) + kb).
+            const int qh = q >> 4;
+            if (~(int8 | skip) & 0xfu) {
+                fp16_scores(buffer, s);
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) s[kb] *= p.score_log2;
+            } else {
+                s[0] = float16v{};
+                s[1] = float16v{};
+            }
+            if (int8) {
+                const float k_factor = k_factor_of(at);
+                int16v acc[2];
+                int8_scores(buffer, acc);
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) {
+                    const bool cell_int8 = (int8 >> (2 * qh + kb)) & 1u;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        s[kb][e] = cell_int8 ? static_cast<float>(acc[kb][e]) * k_factor : s[kb][e];
+                }
+            }
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                if ((skip >> (2 * qh + kb)) & 1u)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) s[kb][e] = -INFINITY;
+        }
+    };
+
+    // ------------------------------------------------------- vector slot
+    auto softmax = [&](const Position& at) TILEMIX_INLINE {
+        const unsigned mode = (at.entry >> Entry::kModeShift) & 3u;
+        pv_pending = mode != Entry::kIdle;
+        // Likewise the probabilities.
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) asm volatile("" : "=v"(ph[ks]));
+        if (!pv_pending) return;
+        float c = p.score_log2;
+        if (mode == Entry::kAllInt8) {
+            c = k_factor_of(at);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                const int16v acc = __builtin_bit_cast(int16v, s[kb]);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) s[kb][e] = static_cast<float>(acc[e]);
+            }
+        } else if (mode == Entry::kMixed) {
+            c = 1.0f;
+        }
+        const unsigned masked = at.entry & Entry::kMasked;
+        if (masked | explicit_scores) {
+            if (c != 1.0f) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) s[kb] *= c;
+                c = 1.0f;
+            }
+            if (masked) {
+                // The last key this lane's row sees, counted from the tile's
+                // first key of the lane.
+                const int k0 = static_cast<int>(at.entry >> Entry::kTileShift) * kTileKeys;
+                int seen = (p.causal ? min(N - 1, qw + q) : N - 1) - k0 - 4 * h;
+                asm volatile("" : "+v"(seen));
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        if (32 * kb + 8 * (e >> 2) + (e & 3) > seen) s[kb][e] = -INFINITY;
+            }
+        }
+        softmax_tile<kOB, false, false>(st, s, c, ph, unused);
+    };
+    // Slot ends: LDS reads done, then the workgroup barrier; with `loads` also
+    // this wave's tile loads.
+    auto slot_end = [&](bool loads) TILEMIX_INLINE {
+        __builtin_amdgcn_sched_barrier(0);
+        if (loads) wait_vmcnt<0>();
+        lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // ----------------------------------------------------------- the walk
+    __syncthreads();
+    load_window();
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    Position now = position(0), next = position(1);
+    issue_k(now.entry, Zero{});
+    slot_end(true);
+    if (second) {
+        // Slot 0: the loads of the first half's slot 0, then its barrier.
+        issue_k(next.entry, One{});
+        issue_v(now.entry, Zero{});
+        slot_end(false);
+    }
+    // Every wave walks `count` positions and passes 2 count + 1 slot ends here;
+    // position x has its tiles in buffers x mod 2.
+    int x = 0;
+    auto walk_position = [&](auto own, auto other) TILEMIX_INLINE {
+        if (!second) {
+            issue_k(next.entry, other);
+            issue_v(now.entry, own);
+        }
+        set_priority<1>();
+        probabilities_times_values(other);
+        scores(now, own);
+        set_priority<0>();
+        const Position after = position(x + 2);
+        slot_end(second);
+        if (second) {
+            issue_k(after.entry, own);
+            issue_v(next.entry, other);
+        }
+        softmax(now);
+        slot_end(!second);
+        now = next;
+        next = after;
+        ++x;
+    };
+    // Two positions a turn; an odd last one is followed by an idle one.
+    while (x < count) {
+        walk_position(Zero{}, One{});
+        walk_position(One{}, Zero{});
+    }
+    probabilities_times_values(One{});
+    if (!second) slot_end(false);
+
+    // ---------------------------------------------------------- epilogue
+    // What only the epilogue needs of the parameters is read again here (the
+    // kernel's first argument), so that it holds no registers during the walk.
+    const auto* late = (const __attribute__((address_space(4))) AttnParams*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    const int dtype = late->o_dtype;
+    const std::int64_t o_row = late->o_row;
+    float a = st.lsum, b = st.lsum;
+    permlane32_swap(a, b);
+    const float l = a + b;
+    const float inverse = l > 0.0f ? 1.0f / l : 0.0f;
+    const int row = qw + q;
+    unsigned char* const Oh = static_cast<unsigned char*>(late->O) + head * late->o_stride * (dtype == TILEMIX_DTYPE_F32 ? 4 : 2);
+    if (dtype == TILEMIX_DTYPE_F32 && d == kDP) {
+        // Stage regions: nobody reads K or K8 any more; at 64 features the
+        // second half also takes the V buffer that the last tile did not use.
+        unsigned char* stage = smem + wave * kStageBytes;
+        if constexpr (2 * L::kKBytes < kWideWaves * kStageBytes) {
+            static_assert(2 * L::kKBytes >= 4 * kStageBytes && 2 * L::kK8Bytes >= 2 * kStageBytes &&
+                              L::kVBytes >= 2 * kStageBytes, "stage regions fit K, K8 and V");
+            if (wave >= 6) stage = smem + kVBase + (wave - 6) * kStageBytes;
+        }
+        store_staged<kOB>(st, stage, reinterpret_cast<float*>(Oh), o_row, inverse, qw, M);
+        return;
+    }
+    if (row < M) {
+        const std::int64_t row_offset = static_cast<std::int64_t>(row) * o_row;
+#pragma unroll
+        for (int fb = 0; fb < kOB; ++fb)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const int feature = (r4 < 2 ? 0 : kDP / 2 - 16) + 16 * fb + 8 * r4 + 4 * h;
+                const float4v value{st.o[fb][4 * r4], st.o[fb][4 * r4 + 1], st.o[fb][4 * r4 + 2], st.o[fb][4 * r4 + 3]};
+                store_output(Oh, dtype, row_offset + feature, value * inverse, d - feature, true);
+            }
     }
 }
 
@@ -1174,15 +1685,25 @@ hipError_t launch_vp(const AttnParams& p, bool precise, hipStream_t stream) {
                    : launch_variant<DC, kPiece, false, kDots, false>(p, stream);
 }
 
+template <int DC>
+hipError_t launch_wide(AttnParams p, hipStream_t stream) {
+    const unsigned blocks = static_cast<unsigned>((p.q_blocks + 1) / 2) * static_cast<unsigned>(p.heads);
+    p.reverse_slots /= 2;  // half as many workgroups, of twice the rows, per XCD
+    attention_wide_kernel<DC><<<blocks, kWideThreads, 0, stream>>>(p);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 // Verification outputs (dots, trace) take the 16-byte or the element kernel.
 // Each head-dimension class DC is compiled in a unit of its own (TILEMIX_DC,
 // set by the build), in parallel; the unit without it holds the host side.
 template <int DC>
-hipError_t launch_dc(const AttnParams& p, int piece, bool precise, hipStream_t stream) {
+hipError_t launch_dc(const AttnParams& p, int piece, bool precise, bool wide, hipStream_t stream) {
     if (p.dots != nullptr || p.trace != nullptr)
         return piece == 16 ? launch_vp<DC, 16, true>(p, precise, stream) : launch_vp<DC, 0, true>(p, precise, stream);
+    if constexpr (DC == 2 || DC == 4)
+        if (wide) return launch_wide<DC>(p, stream);
     switch (piece) {
         case 16: return launch_vp<DC, 16, false>(p, precise, stream);
         case 8: return launch_vp<DC, 8, false>(p, precise, stream);
@@ -1192,13 +1713,13 @@ hipError_t launch_dc(const AttnParams& p, int piece, bool precise, hipStream_t s
 }
 
 #ifdef TILEMIX_DC
-template hipError_t launch_dc<TILEMIX_DC>(const AttnParams&, int, bool, hipStream_t);
+template hipError_t launch_dc<TILEMIX_DC>(const AttnParams&, int, bool, bool, hipStream_t);
 }  // namespace tilemix
 #else
-extern template hipError_t launch_dc<1>(const AttnParams&, int, bool, hipStream_t);
-extern template hipError_t launch_dc<2>(const AttnParams&, int, bool, hipStream_t);
-extern template hipError_t launch_dc<3>(const AttnParams&, int, bool, hipStream_t);
-extern template hipError_t launch_dc<4>(const AttnParams&, int, bool, hipStream_t);
+extern template hipError_t launch_dc<1>(const AttnParams&, int, bool, bool, hipStream_t);
+extern template hipError_t launch_dc<2>(const AttnParams&, int, bool, bool, hipStream_t);
+extern template hipError_t launch_dc<3>(const AttnParams&, int, bool, bool, hipStream_t);
+extern template hipError_t launch_dc<4>(const AttnParams&, int, bool, bool, hipStream_t);
 
 namespace {
 
@@ -1246,11 +1767,35 @@ hipError_t check_device(int* compute_units = nullptr) {
     return supported ? hipSuccess : hipErrorNotSupported;
 }
 
-hipError_t launch_attention(AttnParams p, bool precise, hipStream_t stream) {
+// Whether the wide kernel is the faster one for a launch that it can take
+// (whole 16-byte pieces, head dimensions 33 .. 64 and 97 .. 128, fast P.V, no
+// split, no verification outputs). It halves the tile loads and keeps the
+// matrix cores and exponentials of a CU's two halves apart, but has one
+// workgroup per CU, whose prologue and epilogue nothing overlaps: it needs long
+// walks and whole rounds of workgroups. Rows of a reversed round keep the
+// direction that the 128-row kernel gives them (even number of row blocks).
+// 128-row kernel | wide kernel (us), 64 features: 64 heads x 2048 101.3 | 96.9;
+// 32 x 2048 routed 53.3 | 51.1; 64 x 4096 causal 191.0 | 186.8; 16 x 2048 37.5 |
+// 39.6; 64 x 1024 25.8 | 26.2. 128 features: 32 x 16384 routed 3551 | 3363; 32 x
+// 8192 three-way 847 | 815; 32 x 8192 dense 1064 | 1033, causal 557 | 541; 64 x
+// 4096 causal 320.6 | 315.7; 16 x 4096 causal 106.3 | 108.2; 48 x 3000 (2.25
+// rounds) 258.4 | 263.5; 64 x 1024 46.8 | 48.0; 16 x 2048 48.6 | 53.5. Precise
+// P.V, whose matrix slot is twice as long: 32 x 4096 causal 203.8 | 207.2.
+bool wide_pays(const AttnParams& p, int compute_units) {
+    constexpr int kLongWalk = 32;  // key tiles
+    const int tiles = (p.N - 1) / kTileKeys + 1;
+    if (compute_units <= 0 || tiles < kLongWalk || tiles > kWideMaxTiles) return false;
+    if (p.reverse_slots > 0 && p.q_blocks % 2 != 0) return false;
+    const std::int64_t workgroups = static_cast<std::int64_t>(p.heads) * ((p.q_blocks + 1) / 2);
+    if (p.causal) return workgroups >= 2 * static_cast<std::int64_t>(compute_units);
+    // Whole rounds: at most a tenth of the last one empty.
+    const std::int64_t rounds = (workgroups + compute_units - 1) / compute_units;
+    return 10 * workgroups >= 9 * rounds * compute_units;
+}
+
+// `units`: the device's compute units (check_device).
+hipError_t launch_attention(AttnParams p, int units, bool precise, hipStream_t stream) {
     if (static_cast<long long>(p.q_blocks) * p.heads > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-    int units = 0;
-    hipError_t status = check_device(&units);
-    if (status != hipSuccess) return status;
     // Non-causal heads in the per-XCD head-major order whose query blocks
     // outnumber an XCD's workgroup slots stream K / V once per round of
     // slots; alternate rounds walk the keys in opposite directions.
@@ -1268,11 +1813,12 @@ hipError_t launch_attention(AttnParams p, bool precise, hipStream_t stream) {
     int piece = k_range < (std::int64_t{1} << 31) && v_range < (std::int64_t{1} << 31) ? access_piece(p) : 0;
     if (piece >= 8 && !(p.o_vector && (!p.q8_out || aligned(p.q8_out, 8)))) piece = 4;
     const int dc = (p.d + 31) / 32;
+    const bool wide = piece == 16 && (dc == 2 || dc == 4) && !precise && p.splits <= 1 && !p.dots && !p.trace && wide_pays(p, units);
     switch (dc) {
-        case 1: return launch_dc<1>(p, piece, precise, stream);
-        case 2: return launch_dc<2>(p, piece, precise, stream);
-        case 3: return launch_dc<3>(p, piece, precise, stream);
-        default: return launch_dc<4>(p, piece, precise, stream);
+        case 1: return launch_dc<1>(p, piece, precise, wide, stream);
+        case 2: return launch_dc<2>(p, piece, precise, wide, stream);
+        case 3: return launch_dc<3>(p, piece, precise, wide, stream);
+        default: return launch_dc<4>(p, piece, precise, wide, stream);
     }
 }
 
@@ -1443,7 +1989,7 @@ hipError_t launch_attention_split(AttnParams p, bool precise, const SplitRule& r
     if (found != hipSuccess) return found;
     const int split_tiles = choose_split_tiles(p, precise, units, rule);
     const int device = split_tiles > 0 ? workspace_device(stream) : -1;
-    if (device < 0) return launch_attention(p, precise, stream);
+    if (device < 0) return launch_attention(p, units, precise, stream);
     return with_workspace(device, stream, [&](float* scratch, unsigned*) {
         int tiles = (p.N - 1) / kTileKeys + 1;
         if (p.causal) tiles = std::min(tiles, p.q_blocks * (kRowsPerGroup / kTileKeys));
@@ -1451,7 +1997,7 @@ hipError_t launch_attention_split(AttnParams p, bool precise, const SplitRule& r
         p.splits = (tiles + split_tiles - 1) / split_tiles;
         p.part_o = scratch;
         p.part_ml = scratch + static_cast<std::size_t>(p.heads) * p.splits * p.M * p.d;
-        const hipError_t status = launch_attention(p, precise, stream);
+        const hipError_t status = launch_attention(p, units, precise, stream);
         if (status != hipSuccess) return status;
         const std::int64_t threads = static_cast<std::int64_t>(p.heads) * p.M * ((p.d + 3) / 4);
         const unsigned blocks = static_cast<unsigned>((threads + 255) / 256);
