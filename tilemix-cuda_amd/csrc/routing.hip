@@ -36,6 +36,7 @@ constexpr std::uint8_t kFp16 = TILEMIX_ROUTE_FP16;
 constexpr std::uint8_t kInt8 = TILEMIX_ROUTE_INT8;
 constexpr std::uint8_t kSkip = TILEMIX_ROUTE_SKIP;
 constexpr int kSelectThreads = 1024;
+constexpr std::int64_t kMaxRowWaves = std::int64_t{1} << 22;  // waves of one three-way launch
 constexpr int kMaxSelectEntries = 16384;  // tiles_q + tiles_k kept in LDS by the importance select
 
 __host__ __device__ inline std::uint64_t splitmix64(std::uint64_t x) {
@@ -77,34 +78,46 @@ __global__ void causal_band_kernel(std::uint8_t* codes, int heads, int tiles_q, 
     codes[t] = code;
 }
 
-// One thread per (head, tile row): skip / INT8 / FP16 with probabilities
-// p_skip / p_int8 / rest; a row left entirely skipped gets one tile (column
-// from salt-1 draw of the row) forced FP16.
-__global__ void three_way_kernel(std::uint8_t* codes, int rows, int tiles_k, float p_skip, float p_int8,
-                                 std::uint64_t seed) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
-    std::uint8_t* out = codes + static_cast<std::int64_t>(row) * tiles_k;
-    bool all_skip = true;
-    for (int j = 0; j < tiles_k; ++j) {
-        const float u = uniform24(seed, static_cast<std::uint64_t>(row) * tiles_k + j, 0);
-        const std::uint8_t code = u < p_skip ? kSkip : (u < p_skip + p_int8 ? kInt8 : kFp16);
-        all_skip = all_skip && code == kSkip;
-        out[j] = code;
-    }
-    if (all_skip) {
-        const std::uint64_t h = splitmix64(seed ^ splitmix64(2 * static_cast<std::uint64_t>(row) + 1));
-        out[h % static_cast<std::uint64_t>(tiles_k)] = kFp16;
+// One wave per (head, tile row), lane l drawing tiles l, l + 64, ...: skip /
+// INT8 / FP16 with probabilities p_skip / p_int8 / rest; a row left entirely
+// skipped gets one tile (column from the salt-1 draw of the row) forced FP16,
+// by the lane that stored that tile. A draw is two rounds of 64-bit
+// multiplies, so a row per thread was a serial chain of tiles_k draws on a
+// few waves, its byte stores tiles_k apart: with the packer, 32 heads x 128
+// rows x 256 tiles took 35.1 us per pass and now take 15.9, the time of two
+// launches (as 64 heads x 5 x 10 did and do).
+__global__ __launch_bounds__(256) void three_way_kernel(std::uint8_t* codes, int rows, int tiles_k, float p_skip,
+                                                        float p_int8, std::uint64_t seed) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int waves = static_cast<int>(gridDim.x) * (256 / kWave);
+    for (std::int64_t row = blockIdx.x * (256 / kWave) + threadIdx.x / kWave; row < rows; row += waves) {
+        std::uint8_t* out = codes + row * tiles_k;
+        bool all_skip = true;
+        for (int j = lane; j < tiles_k; j += kWave) {
+            const float u = uniform24(seed, static_cast<std::uint64_t>(row) * tiles_k + j, 0);
+            const std::uint8_t code = u < p_skip ? kSkip : (u < p_skip + p_int8 ? kInt8 : kFp16);
+            all_skip = all_skip && code == kSkip;
+            out[j] = code;
+        }
+        if (__ballot(!all_skip) == 0) {
+            const std::uint64_t h = splitmix64(seed ^ splitmix64(2 * static_cast<std::uint64_t>(row) + 1));
+            const int forced = static_cast<int>(h % static_cast<std::uint64_t>(tiles_k));
+            if ((forced & (kWave - 1)) == lane) out[forced] = kFp16;
+        }
     }
 }
 
 // Absolute maximum of each tile row block of Q (blockIdx.x < tiles_q) and
 // each key block of K (the rest), per head (blockIdx.y): amax[head][tiles_q +
-// tiles_k]. NaN elements are passed over, as fmaxf does. kVector (d % 8 == 0,
-// 16-byte aligned heads): 16-byte loads and the maximum over fp16 bit
-// patterns with the sign cleared (unsigned order is value order for them;
-// NaN patterns sort above +inf, so a maximum above 0x7c00 sends the block
-// through a second pass that leaves NaNs out).
+// tiles_k]. NaN elements are passed over, as fmaxf does. kVector (dword-aligned
+// heads, so that every block's 16-byte loads are: a block starts a multiple of
+// 16 rows into its head): 16-byte loads, the fewer than 8 elements past the
+// last whole one by themselves, and the maximum over fp16 bit patterns with
+// the sign cleared (unsigned order is value order for them; NaN patterns sort
+// above +inf, so a maximum above 0x7c00 sends the block through a second pass
+// that leaves NaNs out). Memory bound; the element-wise form stays for heads at
+// an odd 2-byte address. Router and packer over 32 heads x 16383 x 100 (d % 8
+// != 0, once element-wise): 133.7 -> 58.2 us; 16384 x 128: 67.8 before and after.
 template <bool kVector>
 __global__ __launch_bounds__(256) void tile_absmax_kernel(const std::uint16_t* Q, const std::uint16_t* K, int M,
                                                           int N, int d, std::int64_t q_stride,
@@ -132,13 +145,14 @@ __global__ __launch_bounds__(256) void tile_absmax_kernel(const std::uint16_t* Q
 #pragma unroll
             for (int u = 0; u < kLoads; ++u) {
                 const std::int64_t c = base + u * 256;
-                v[u] = c < chunks ? *reinterpret_cast<const uint4v*>(x + 8 * c) : uint4v{0u, 0u, 0u, 0u};
+                v[u] = c < chunks ? *reinterpret_cast<const uint4v_dword*>(x + 8 * c) : uint4v{0u, 0u, 0u, 0u};
             }
 #pragma unroll
             for (int u = 0; u < kLoads; ++u)
 #pragma unroll
                 for (int w = 0; w < 4; ++w) top = max_u16x2(top, v[u][w] & 0x7fff7fffu);
         }
+        if (threadIdx.x < count % 8) top = max_u16x2(top, x[8 * chunks + threadIdx.x] & 0x7fffu);
         unsigned bits = wave_max_bits(max(top & 0xffffu, top >> 16));
         if ((threadIdx.x & (kWave - 1)) == 0) partial_bits[threadIdx.x / kWave] = bits;
         __syncthreads();
@@ -520,7 +534,9 @@ extern "C" int tilemix_tiles_three_way(std::uint8_t* tile_codes, int heads, int 
     const int tiles_q = (M - 1) / tile_rows + 1, tiles_k = (N - 1) / tile_keys + 1;
     const std::int64_t rows = static_cast<std::int64_t>(heads) * tiles_q;
     if (rows > 0x7fffffff || !grid_ok(rows, 256)) return hipErrorInvalidConfiguration;
-    three_way_kernel<<<blocks_for(rows, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
+    // A wave per row, and further rounds past 2^22 rows: a grid holds fewer than 2^32 threads.
+    const std::int64_t waves = rows < kMaxRowWaves ? rows : kMaxRowWaves;
+    three_way_kernel<<<blocks_for(waves * kWave, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(
         tile_codes, static_cast<int>(rows), tiles_k, p_skip, p_int8, seed);
     return hipGetLastError();
 }
@@ -604,8 +620,8 @@ hipError_t launch_importance(const std::uint16_t* Q, const std::uint16_t* K, int
     const std::int64_t qs = heads > 1 ? q_head_stride : static_cast<std::int64_t>(M) * d;
     const std::int64_t ks = heads > 1 ? k_head_stride : static_cast<std::int64_t>(N) * d;
     const dim3 grid(static_cast<unsigned>(tiles_q + tiles_k), static_cast<unsigned>(heads));
-    const bool vector = d % 8 == 0 && reinterpret_cast<std::uintptr_t>(Q) % 16 == 0 &&
-                        reinterpret_cast<std::uintptr_t>(K) % 16 == 0 && (qs * 2) % 16 == 0 && (ks * 2) % 16 == 0;
+    const bool vector = reinterpret_cast<std::uintptr_t>(Q) % 4 == 0 && reinterpret_cast<std::uintptr_t>(K) % 4 == 0 &&
+                        qs % 2 == 0 && ks % 2 == 0;
     if (vector)
         tile_absmax_kernel<true><<<grid, 256, 0, s>>>(Q, K, M, N, d, qs, ks, tiles_q, tiles_k, tile_rows, tile_keys,
                                                       workspace);

@@ -22,6 +22,7 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef unsigned int uint4v __attribute__((ext_vector_type(4)));
 typedef unsigned int uint2v __attribute__((ext_vector_type(2)));
+typedef uint4v uint4v_dword __attribute__((aligned(4)));  // in memory at any dword address
 typedef __attribute__((address_space(3))) short4v lds_short4v;
 
 inline constexpr int kWave = 64;
