@@ -3,13 +3,13 @@
 // Replaces quantize_tilemix_qk / quantize_blocks<BlockRows> of the reference
 // (src/tilemix.cu:16-49, 223-236). One 256-thread workgroup owns one
 // quantization block (128 Q rows or 64 K rows x d features). Because rows are
-// contiguous, a block is one contiguous span of rows*d halves: the vector path
-// reads it once with 16-byte loads into registers (at most 8 per thread),
-// reduces the absmax across the workgroup and quantizes from registers, so HBM
-// sees exactly one read of the input and one write of the int8 output. The
-// absmax runs on packed fp16 pairs (magnitudes by clearing the sign bits) and
-// the per-element quotient uses the block's reciprocal with an exact
-// correction step instead of a division (quantize_value_recip).
+// contiguous, a block is one contiguous span of rows*d halves: the piece paths
+// read it once with 16-byte or 8-byte loads into registers (at most 64 halves
+// per thread), reduce the absmax across the workgroup and quantize from
+// registers, so HBM sees exactly one read of the input and one write of the
+// int8 output. The absmax runs on packed fp16 pairs (magnitudes by clearing the
+// sign bits) and the per-element quotient uses the block's reciprocal with an
+// exact correction step instead of a division (quantize_value_recip).
 
 #include "tilemix_device.h"
 #include "tilemix_launch.h"
@@ -20,13 +20,32 @@ namespace tilemix {
 namespace {
 
 constexpr int kQuantThreads = 256;
-constexpr int kQuantMaxChunks = (128 * 128 / 8) / kQuantThreads;  // 16-byte chunks per thread
+constexpr int kQuantMaxElements = 128 * 128;  // of a block: 64 per thread
 
+template <int kPiece>
+struct PieceTypes;  // kPiece fp16 values in, kPiece bytes out
+template <>
+struct PieceTypes<8> {
+    typedef uint4v Halves;
+    typedef uint2v Bytes;
+};
+template <>
+struct PieceTypes<4> {
+    typedef uint2v Halves;
+    typedef std::uint32_t Bytes;
+};
+
+// kPiece: elements a load takes, 0 for the element-wise form. Pieces of 8 are
+// 16-byte loads of rows that are whole and 16-byte aligned in them; pieces of
+// 4, 8-byte loads, take the other rows that are multiples of 4 elements and
+// 8-byte aligned (d = 100, 36, or d = 128 at a row stride of 132). HBM bound:
+// 64 heads x 4096 x 100 in pieces of 4 31.4 us (157 MB, 5.0 TB/s), element by
+// element 131.1 us; in pieces of 8 x 128 37.9 us (201 MB, 5.3 TB/s).
 // kContiguous: rows are d elements apart, so a block is one span of
-// rows * d halves; otherwise chunk c of the block is chunk c % (d / 8) of row
-// c / (d / 8). kChunks: 16-byte chunks held per thread, enough for the
-// larger block of the launch (4 for 64 x 128 K blocks, 8 for 128 x 128 Q).
-template <bool kVector, bool kContiguous, int kChunks = kQuantMaxChunks>
+// rows * d halves; otherwise piece c of the block is piece c % (d / kPiece) of
+// row c / (d / kPiece). kPieces: pieces held per thread, enough for the larger
+// block of the launch (4 of 8 for 64 x 128 K blocks, 8 for 128 x 128 Q).
+template <int kPiece, bool kContiguous, int kPieces>
 __global__ __launch_bounds__(kQuantThreads) void quantize_blocks_kernel(QuantSide q, QuantSide k, int d) {
     __shared__ float partial[kQuantThreads / kWave];
     __shared__ unsigned partial_bits[kQuantThreads / kWave];
@@ -43,32 +62,34 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_blocks_kernel(QuantSid
                        static_cast<std::int64_t>(first) * d;
     const int t = threadIdx.x;
 
-    uint4v chunk[kChunks];
-    const int chunks = count / 8;
     float absmax = 0.0f;
-    if constexpr (kVector) {
-        // Chunks past the block's end load its last chunk again (in-block
+    constexpr int kWords = kPiece ? kPiece / 2 : 1;  // 32-bit words of a piece
+    using Types = PieceTypes<kPiece ? kPiece : 8>;
+    typename Types::Halves piece[kPieces];
+    const int pieces = kPiece ? count / (kPiece ? kPiece : 1) : 0;
+    if constexpr (kPiece > 0) {
+        // Pieces past the block's end load its last piece again (in-block
         // values, which leave the maximum unchanged; they are not stored).
+        const int per_row = d / kPiece;
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
+        for (int c = 0; c < kPieces; ++c) {
             const int index = t + c * kQuantThreads;
-            const int at = index < chunks ? index : chunks - 1;
+            const int at = index < pieces ? index : pieces - 1;
             const std::uint16_t* source;
             if constexpr (kContiguous) {
-                source = in + 8 * at;
+                source = in + kPiece * at;
             } else {
-                const int per_row = d / 8;
-                source = in + (at / per_row) * row_stride + 8 * (at % per_row);
+                source = in + (at / per_row) * row_stride + kPiece * (at % per_row);
             }
-            chunk[c] = *reinterpret_cast<const uint4v*>(source);
+            piece[c] = *reinterpret_cast<const typename Types::Halves*>(source);
         }
         // |x| as fp16 bit patterns: unsigned order is float order for them,
         // NaN patterns (> 0x7c00) sorting above +inf.
         unsigned top = 0;
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c)
+        for (int c = 0; c < kPieces; ++c)
 #pragma unroll
-            for (int w = 0; w < 4; ++w) top = max_u16x2(top, chunk[c][w] & 0x7fff7fffu);
+            for (int w = 0; w < kWords; ++w) top = max_u16x2(top, piece[c][w] & 0x7fff7fffu);
         unsigned bits = wave_max_bits(max(top & 0xffffu, top >> 16));
         if ((t & (kWave - 1)) == 0) partial_bits[t / kWave] = bits;
         __syncthreads();
@@ -77,10 +98,10 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_blocks_kernel(QuantSid
             // A NaN in the block: the maximum skips NaNs, as fmaxf does.
             unsigned clean = 0;
 #pragma unroll
-            for (int c = 0; c < kChunks; ++c)
+            for (int c = 0; c < kPieces; ++c)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const unsigned h = (chunk[c][e / 2] >> (16 * (e % 2))) & 0x7fffu;
+                for (int e = 0; e < kPiece; ++e) {
+                    const unsigned h = (piece[c][e / 2] >> (16 * (e % 2))) & 0x7fffu;
                     clean = h <= 0x7c00u ? max(clean, h) : clean;
                 }
             clean = wave_max_bits(clean);
@@ -102,29 +123,33 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_blocks_kernel(QuantSid
     const float recip = 1.0f / scale;  // used only when scale > 0
     if (t == 0) side.scales[head * side.blocks + block] = float_to_half_bits(scale);
 
-    if constexpr (kVector) {
+    if constexpr (kPiece > 0) {
         if (scale > 0.0f) {
 #pragma unroll
-            for (int c = 0; c < kChunks; ++c) {
+            for (int c = 0; c < kPieces; ++c) {
                 const int index = t + c * kQuantThreads;
-                if (index < chunks) {
-                    int v[8];
+                if (index < pieces) {
+                    int v[kPiece];
 #pragma unroll
-                    for (int e = 0; e < 8; e += 2) {
-                        v[e] = quantize_half<0>(chunk[c][e / 2], scale, recip);
-                        v[e + 1] = quantize_half<1>(chunk[c][e / 2], scale, recip);
+                    for (int e = 0; e < kPiece; e += 2) {
+                        v[e] = quantize_half<0>(piece[c][e / 2], scale, recip);
+                        v[e + 1] = quantize_half<1>(piece[c][e / 2], scale, recip);
                     }
-                    uint2v packed;
-                    packed[0] = pack_bytes(v[0], v[1], v[2], v[3]);
-                    packed[1] = pack_bytes(v[4], v[5], v[6], v[7]);
-                    reinterpret_cast<uint2v*>(out)[index] = packed;
+                    typename Types::Bytes packed;
+                    if constexpr (kPiece == 8) {
+                        packed[0] = pack_bytes(v[0], v[1], v[2], v[3]);
+                        packed[1] = pack_bytes(v[4], v[5], v[6], v[7]);
+                    } else {
+                        packed = pack_bytes(v[0], v[1], v[2], v[3]);
+                    }
+                    reinterpret_cast<typename Types::Bytes*>(out)[index] = packed;
                 }
             }
         } else {
 #pragma unroll
-            for (int c = 0; c < kChunks; ++c) {
+            for (int c = 0; c < kPieces; ++c) {
                 const int index = t + c * kQuantThreads;
-                if (index < chunks) reinterpret_cast<uint2v*>(out)[index] = uint2v{0u, 0u};
+                if (index < pieces) reinterpret_cast<typename Types::Bytes*>(out)[index] = typename Types::Bytes{};
             }
         }
     } else {
@@ -138,6 +163,22 @@ bool aligned(const void* pointer, std::size_t bytes) {
     return (reinterpret_cast<std::uintptr_t>(pointer) % bytes) == 0;
 }
 
+// Whether the rows of a side move in pieces of `piece` elements: rows that are
+// whole in them, at addresses that are multiples of a piece. With d % piece ==
+// 0 every block's bytes start at a multiple of `piece` too.
+bool takes_pieces(const QuantSide& side, int d, int piece) {
+    return side.blocks == 0 || (d % piece == 0 && aligned(side.x, 2 * piece) && aligned(side.x8, piece) &&
+                                side.in_head_stride % piece == 0 && side.in_row_stride % piece == 0);
+}
+
+template <int kPiece, int kPieces>
+void launch_pieces(bool contiguous, dim3 grid, hipStream_t stream, const QuantSide& q, const QuantSide& k, int d) {
+    if (contiguous)
+        quantize_blocks_kernel<kPiece, true, kPieces><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+    else
+        quantize_blocks_kernel<kPiece, false, kPieces><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+}
+
 }  // namespace
 
 hipError_t launch_quantize(const QuantSide& q, const QuantSide& k, int heads, int d,
@@ -145,32 +186,29 @@ hipError_t launch_quantize(const QuantSide& q, const QuantSide& k, int heads, in
     const int blocks = q.blocks + k.blocks;
     if (blocks == 0) return hipSuccess;
     if (heads > 65535) return hipErrorInvalidConfiguration;
-    // The vector path reads 16-byte chunks of halves and writes 8-byte chunks
-    // of int8; rows of d % 8 == 0 halves keep every block start aligned.
-    bool vector = d % 8 == 0;
     bool contiguous = true;
+    int most_rows = 0;  // of a block of the launch
     for (const QuantSide* side : {&q, &k}) {
         if (side->blocks == 0) continue;
-        vector = vector && aligned(side->x, 16) && aligned(side->x8, 8) &&
-                 (side->in_head_stride * 2) % 16 == 0 && (side->in_row_stride * 2) % 16 == 0;
         contiguous = contiguous && side->in_row_stride == d;
+        most_rows = std::max(most_rows, side->block_rows);
     }
     const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(heads));
-    // Chunks of 16 bytes per thread the larger block of the launch needs.
-    std::int64_t need = 0;
-    for (const QuantSide* side : {&q, &k})
-        if (side->blocks) need = std::max<std::int64_t>(need, static_cast<std::int64_t>(side->block_rows) * d / 8);
-    const bool small = need <= 4 * kQuantThreads;
-    if (vector && contiguous && small)
-        quantize_blocks_kernel<true, true, 4><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
-    else if (vector && contiguous)
-        quantize_blocks_kernel<true, true><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
-    else if (vector && small)
-        quantize_blocks_kernel<true, false, 4><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
-    else if (vector)
-        quantize_blocks_kernel<true, false><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
-    else
-        quantize_blocks_kernel<false, false><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+    // Registers for half of the largest block where that is enough.
+    const bool small = most_rows * d <= kQuantMaxElements / 2;
+    if (takes_pieces(q, d, 8) && takes_pieces(k, d, 8)) {
+        if (small)
+            launch_pieces<8, kQuantMaxElements / 2 / 8 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+        else
+            launch_pieces<8, kQuantMaxElements / 8 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+    } else if (takes_pieces(q, d, 4) && takes_pieces(k, d, 4)) {
+        if (small)
+            launch_pieces<4, kQuantMaxElements / 2 / 4 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+        else
+            launch_pieces<4, kQuantMaxElements / 4 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+    } else {
+        quantize_blocks_kernel<0, false, 1><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+    }
     return hipGetLastError();
 }
 
