@@ -48,3 +48,30 @@ def test_pieces_match_oracle(tm, oracle_lib, cuda, heads, M, N, d, pad, shift, s
         check_side(oracle_lib, x, host(out)[:x.size].reshape(x.shape), host(s, np.uint16), block, label)
         whole = host(flat)
         assert (whole[:shift8] == -128).all() and (whole[-GUARD:] == -128).all(), f"{label}: written past its end"
+
+
+@pytest.mark.parametrize("heads,M,N,d,pad", [
+    (3, 300, 200, 128, 0), (5, 129, 65, 64, 0), (2, 130, 1, 128, 64),  # the grid runs over heads first
+    (3, 300, 200, 96, 0), (3, 300, 200, 64, 8), (3, 300, 200, 100, 0),  # over blocks first
+    (1, 300, 200, 128, 0),
+])
+def test_interleaved_heads_match_oracle(tm, oracle_lib, cuda, heads, M, N, d, pad):
+    """[rows, heads, d + pad] inputs, both grid orders."""
+    import torch
+
+    print(f"quantizer interleaved heads={heads} M={M} N={N} d={d} pad={pad}", flush=True)
+    rng = np.random.default_rng(M * d + pad)
+    row = heads * (d + pad)
+    inputs, ins, outs, scales = [], [], [], []
+    for rows, block in ((M, 128), (N, 64)):
+        inputs.append(np.stack([special_rows(rows, d, block, rng) for _ in range(heads)]))
+        wide = np.full((rows, heads, d + pad), 0x7C00, np.uint16)
+        wide[:, :, :d] = inputs[-1].transpose(1, 0, 2)
+        ins.append(dev_half(wide))
+        outs.append(torch.full((heads, rows, d), -128, dtype=torch.int8, device=cuda))
+        scales.append(torch.full((heads, -(-rows // block)), 0x7B53, dtype=torch.int16, device=cuda))
+    tm.check(tm.quantize_tilemix_qk_strided(ins[0], ins[1], outs[0], outs[1], scales[0], scales[1], heads, M, N, d,
+                                            d + pad, d + pad, row, row))
+    torch.cuda.synchronize()
+    for x, out, s, block, label in zip(inputs, outs, scales, (128, 64), "QK"):
+        check_side(oracle_lib, x, host(out), host(s, np.uint16), block, label)

@@ -21,6 +21,7 @@ namespace {
 
 constexpr int kQuantThreads = 256;
 constexpr int kQuantMaxElements = 128 * 128;  // of a block: 64 per thread
+constexpr int kLineHalves = 64;  // fp16 values of a 128-byte cache line
 
 template <int kPiece>
 struct PieceTypes;  // kPiece fp16 values in, kPiece bytes out
@@ -45,14 +46,17 @@ struct PieceTypes<4> {
 // rows * d halves; otherwise piece c of the block is piece c % (d / kPiece) of
 // row c / (d / kPiece). kPieces: pieces held per thread, enough for the larger
 // block of the launch (4 of 8 for 64 x 128 K blocks, 8 for 128 x 128 Q).
+// heads_first: the grid is [heads, blocks] instead of [blocks, heads].
 template <int kPiece, bool kContiguous, int kPieces>
-__global__ __launch_bounds__(kQuantThreads) void quantize_blocks_kernel(QuantSide q, QuantSide k, int d) {
+__global__ __launch_bounds__(kQuantThreads) void quantize_blocks_kernel(QuantSide q, QuantSide k, int d,
+                                                                            bool heads_first) {
     __shared__ float partial[kQuantThreads / kWave];
     __shared__ unsigned partial_bits[kQuantThreads / kWave];
-    const bool is_q = static_cast<int>(blockIdx.x) < q.blocks;
+    const int at_block = static_cast<int>(heads_first ? blockIdx.y : blockIdx.x);
+    const bool is_q = at_block < q.blocks;
     const QuantSide side = is_q ? q : k;
-    const int block = is_q ? static_cast<int>(blockIdx.x) : static_cast<int>(blockIdx.x) - q.blocks;
-    const std::int64_t head = blockIdx.y;
+    const int block = is_q ? at_block : at_block - q.blocks;
+    const std::int64_t head = heads_first ? blockIdx.x : blockIdx.y;
     const int first = block * side.block_rows;
     const int last = min(side.rows, first + side.block_rows);
     const int count = (last - first) * d;
@@ -172,11 +176,12 @@ bool takes_pieces(const QuantSide& side, int d, int piece) {
 }
 
 template <int kPiece, int kPieces>
-void launch_pieces(bool contiguous, dim3 grid, hipStream_t stream, const QuantSide& q, const QuantSide& k, int d) {
+void launch_pieces(bool contiguous, bool heads_first, dim3 grid, hipStream_t stream, const QuantSide& q,
+                   const QuantSide& k, int d) {
     if (contiguous)
-        quantize_blocks_kernel<kPiece, true, kPieces><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+        quantize_blocks_kernel<kPiece, true, kPieces><<<grid, kQuantThreads, 0, stream>>>(q, k, d, heads_first);
     else
-        quantize_blocks_kernel<kPiece, false, kPieces><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+        quantize_blocks_kernel<kPiece, false, kPieces><<<grid, kQuantThreads, 0, stream>>>(q, k, d, heads_first);
 }
 
 }  // namespace
@@ -187,27 +192,36 @@ hipError_t launch_quantize(const QuantSide& q, const QuantSide& k, int heads, in
     if (blocks == 0) return hipSuccess;
     if (heads > 65535) return hipErrorInvalidConfiguration;
     bool contiguous = true;
+    bool heads_first = d % kLineHalves == 0 && blocks <= 65535;
     int most_rows = 0;  // of a block of the launch
     for (const QuantSide* side : {&q, &k}) {
         if (side->blocks == 0) continue;
         contiguous = contiguous && side->in_row_stride == d;
+        heads_first = heads_first && side->in_head_stride < side->in_row_stride &&
+                      side->in_head_stride % kLineHalves == 0;
         most_rows = std::max(most_rows, side->block_rows);
     }
-    const dim3 grid(static_cast<unsigned>(blocks), static_cast<unsigned>(heads));
+    // Workgroups that run together read memory that lies together: the blocks of
+    // a head in turn, or where rows hold all heads ([rows, heads, d]) the heads
+    // of a block: 64 heads x 4096 x 128 46.5 -> 41.1 us, 8 x 16384 x 128 20.1 ->
+    // 19.7, 64 x 4096 x 64 20.9 both ways. Heads that share cache lines keep the
+    // first order: 32 x 4096 x 100 17.3 us against 19.4.
+    const dim3 grid(static_cast<unsigned>(heads_first ? heads : blocks),
+                    static_cast<unsigned>(heads_first ? blocks : heads));
     // Registers for half of the largest block where that is enough.
     const bool small = most_rows * d <= kQuantMaxElements / 2;
     if (takes_pieces(q, d, 8) && takes_pieces(k, d, 8)) {
         if (small)
-            launch_pieces<8, kQuantMaxElements / 2 / 8 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+            launch_pieces<8, kQuantMaxElements / 2 / 8 / kQuantThreads>(contiguous, heads_first, grid, stream, q, k, d);
         else
-            launch_pieces<8, kQuantMaxElements / 8 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+            launch_pieces<8, kQuantMaxElements / 8 / kQuantThreads>(contiguous, heads_first, grid, stream, q, k, d);
     } else if (takes_pieces(q, d, 4) && takes_pieces(k, d, 4)) {
         if (small)
-            launch_pieces<4, kQuantMaxElements / 2 / 4 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+            launch_pieces<4, kQuantMaxElements / 2 / 4 / kQuantThreads>(contiguous, heads_first, grid, stream, q, k, d);
         else
-            launch_pieces<4, kQuantMaxElements / 4 / kQuantThreads>(contiguous, grid, stream, q, k, d);
+            launch_pieces<4, kQuantMaxElements / 4 / kQuantThreads>(contiguous, heads_first, grid, stream, q, k, d);
     } else {
-        quantize_blocks_kernel<0, false, 1><<<grid, kQuantThreads, 0, stream>>>(q, k, d);
+        quantize_blocks_kernel<0, false, 1><<<grid, kQuantThreads, 0, stream>>>(q, k, d, heads_first);
     }
     return hipGetLastError();
 }
