@@ -7,6 +7,7 @@
 * quant_division_check runs the quantizer's division-free quotient against
   IEEE division for every fp16 (block maximum, value) pair, compiled with the
   library's own device flags.
+* launch_rules checks the library's launch rules on the CPU (host code only).
 
 Usage: python tests/native/build.py
 """
@@ -23,6 +24,7 @@ ROOT = HERE.parent.parent
 OUT = HERE / "_build"
 EXE = OUT / "tilemix_native"
 DIVISION_CHECK = OUT / "quant_division_check"
+LAUNCH_RULES = OUT / "launch_rules"
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 
 
@@ -64,6 +66,16 @@ def build_division_check() -> Path:
           f"-I{library_build.CSRC}", str(HERE / "quant_division_check.hip"), "-o", str(tmp)])
     os.replace(tmp, DIVISION_CHECK)
     return DIVISION_CHECK
+
+
+def build_launch_rules() -> Path:
+    library_build = _library_build()
+    OUT.mkdir(parents=True, exist_ok=True)
+    tmp = LAUNCH_RULES.with_suffix(".tmp")
+    _run([HIPCC, "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-Wno-unused-command-line-argument",
+          f"-I{ROOT / 'include'}", f"-I{library_build.CSRC}", str(HERE / "launch_rules.cpp"), "-o", str(tmp)])
+    os.replace(tmp, LAUNCH_RULES)
+    return LAUNCH_RULES
 
 
 if __name__ == "__main__":

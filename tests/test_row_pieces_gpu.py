@@ -29,6 +29,8 @@ CASES = [
     (2, 90, 129, 4, 1, False, False, 1, 0), (2, 200, 200, 128, 2, True, False, 1, 2), (2, 150, 129, 64, 1, False, True, 0, 2),
     (2, 100, 200, 72, 1, False, False, 1, 4), (2, 100, 200, 96, 1, False, True, 1, 1), (1, 300, 700, 88, 2, False, True, 1, 0),
     (2, 120, 100, 22, 1, False, False, 1, 0),
+    # K8 rows of 4 bytes: pieces of the tile before the last that would end past the head
+    (2, 70, 65, 4, 1, False, False, 1, 0), (3, 130, 194, 4, 2, False, True, 2, 0), (2, 90, 131, 4, 1, False, False, 0, 0),
 ]
 
 

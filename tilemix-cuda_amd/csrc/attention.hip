@@ -516,8 +516,9 @@ __device__ __forceinline__ void prepare_q(const AttnParams& p, std::int64_t head
 // start on 8 bytes, in 16-byte pieces from dword-aligned addresses; a row's
 // last piece may carry the next row's first bytes, which meet zeros of Q8. 4:
 // K and V rows too; what a K row's last piece carries past d is masked when it
-// is read (V's reaches only features past d of O). A piece that would end past
-// the head comes in by dwords instead (load_tile_dwords). 0: single elements.
+// is read (V's reaches only features past d of O). A tile of which a piece would
+// end past the head comes in by dwords instead (load_tile_dwords). 0: single
+// elements.
 // kSplit: the workgroup covers one range of key tiles of its 128-row block
 // and writes that range's partial row state (AttnParams::splits).
 template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
@@ -695,9 +696,10 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 load_to_lds(r, dst_v[t] == lds_spare_address ? dst_v[t] : dst_v[t] + shift, off_v[t], soffset);
         }
     };
-    // A tile whose rows are not whole 16-byte pieces and that reaches the
-    // head's last row (whose last piece would end past the head): dwords
-    // through registers, zeros past d and N. at(row, byte): the LDS position.
+    // A tile whose rows are not whole 16-byte pieces and of which a piece would
+    // end past the head (that of the head's last row, and for K8 rows of four
+    // bytes that of up to three rows before it): dwords through registers,
+    // zeros past d and N. at(row, byte): the LDS position.
     auto load_tile_dwords = [&](unsigned char* tile, const unsigned char* head_rows, std::int64_t row_bytes, int k0,
                                 int valid_bytes, int padded_bytes, auto&& at) {
         const int per_row = padded_bytes / 4;
@@ -723,7 +725,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
                 else k_slots(rsrc_k, k0 * k_row_bytes);
             }
             if (need8) {
-                if (kPiece != 16 && last)
+                if (kPiece != 16 && (last || (kPiece == 4 && k8_pieces_pass_end(k0, N, d))))
                     load_tile_dwords(lds_k8, reinterpret_cast<const unsigned char*>(K8h), d, k0, d, L::kDP8,
                                      [](int row, int byte) { return L::k8_at(row, byte); });
                 else if (tail) k8_slots(rsrc_from(rsrc_k8, k0 * d), 0);

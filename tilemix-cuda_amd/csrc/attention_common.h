@@ -339,6 +339,15 @@ inline int access_piece(const AttnParams& p) {
     return 0;
 }
 
+// Whether 16-byte pieces of int8 rows, `d` bytes long and apart, of the key tile
+// at k0 reach past the last of N rows. A row's last piece carries up to 12 bytes
+// of what follows the row: one more row holds them unless d is 4, where it takes
+// three. (The range check of a piece covers its lane's offset but not the tile's.)
+__host__ __device__ constexpr bool k8_pieces_pass_end(int k0, int N, int d) {
+    const std::int64_t last_row = k0 + kTileKeys < N ? k0 + kTileKeys - 1 : N - 1;
+    return last_row * d + (d + 15) / 16 * 16 > static_cast<std::int64_t>(N) * d;
+}
+
 // decode.hip: M <= kMaxDecodeRows query rows per head. decode_worthwhile:
 // whether it is the faster kernel for the call; plan_decode: workgroups
 // per head for a workspace of scratch_floats and max_arrivals counters (1:
