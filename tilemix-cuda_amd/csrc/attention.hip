@@ -561,10 +561,10 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     const int M = p.M, N = p.N, d = p.d;
     const std::int64_t part = kSplit ? (head * p.splits + split) * M : 0;  // this split's first partial row
     if constexpr (kSplit && !kDots) {
-        // A range that lies past the block's causal diagonal: no key.
+        // A range that lies past the block's causal diagonal: no key, no O.
         if (p.causal && split * p.split_tiles * kTileKeys > q0 + kRowsPerGroup - 1) {
             if (tid < kRowsPerGroup && q0 + tid < M)
-                *reinterpret_cast<float2v*>(p.part_ml + 2 * (part + q0 + tid)) = float2v{-INFINITY, 0.0f};
+                *reinterpret_cast<float2v*>(p.part_ml + 2 * (part + q0 + tid)) = float2v{-INFINITY, kNoPart};
             return;
         }
     }
@@ -1608,15 +1608,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void attention_wide_kernel(const A
     }
 }
 
-// O of a key-range split launch: per row, m = max over the splits of m_s,
-// O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s (log2-domain row states;
-// splits whose rows saw no key have m_s = -inf and weigh nothing; of those
-// past a causal diagonal only the row states are written). One thread per
-// head, row and 4 features, splits summed in order. Splits are taken kBatch at
-// a time, every load of a batch issued before any use (one memory round trip
-// per batch); m is the maximum over the splits seen so far, and a later batch
-// that raises it rescales the sums (up to kBatch splits: one batch, m over all
-// splits).
+// O of a key-range split launch: each row's parts merged (merge_part), splits in
+// order; those past a causal diagonal hold a state only (kNoPart). One thread
+// per head, row and 4 features. Splits are taken kBatch at a time, every load of
+// a batch issued before any use (one memory round trip per batch).
 template <bool kVector>
 __global__ __launch_bounds__(256) void split_combine_kernel(const AttnParams p) {
     constexpr int kBatch = 16;
@@ -1645,24 +1640,13 @@ __global__ __launch_bounds__(256) void split_combine_kernel(const AttnParams p) 
                 for (int e = 0; e < 4; ++e) value[b][e] = f0 + e < d ? src[e] : 0.0f;
             }
         }
-        float m_next = m;
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b)
-            if (s0 + b < splits) m_next = fmaxf(m_next, state[b][0]);
-        if (m_next == -INFINITY) continue;  // no split so far saw a key of this row
-        if (m_next != m) {
-            const float rescale = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_next);
-            l *= rescale;
-            acc *= rescale;
-            m = m_next;
-        }
 #pragma unroll
         for (int b = 0; b < kBatch; ++b) {
-            const bool counts = s0 + b < splits && state[b][0] != -INFINITY;
-            const float w = counts ? __builtin_amdgcn_exp2f(state[b][0] - m) : 0.0f;
-            l += w * state[b][1];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] += w * (counts ? value[b][e] : 0.0f);
+            if (s0 + b < splits) {
+                const bool there = state[b][1] != kNoPart;
+                const PartWeights w = merge_part(m, l, there ? state[b][0] : -INFINITY, there ? state[b][1] : 0.0f);
+                acc = merged(acc, there ? value[b] : float4v{0.0f, 0.0f, 0.0f, 0.0f}, w);
+            }
         }
     }
     const float inverse = l > 0.0f ? 1.0f / l : 0.0f;

@@ -249,6 +249,35 @@ __device__ __forceinline__ void set_priority() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Merge of a row's parts (log2-domain maximum, sum, unnormalised O; one part per
+// range of keys), in the order of the ranges. merge_part takes the part's state
+// into (m, l), and with the weights that it returns merged() takes its O. The
+// side with the larger maximum keeps weight 1, so a part costs one exponential.
+// A part of maximum -inf weighs 0 beside finite ones, by multiplication: it may
+// have seen keys whose scores are all NaN (a NaN in its query row), and its sum
+// and O are NaN then, which the row has to become. One that was never written
+// has the sum kNoPart; the caller puts a state of (-inf, 0) and O = 0 in its place.
+struct PartWeights {
+    float keep;  // of what is merged so far
+    float part;
+};
+inline constexpr float kNoPart = -1.0f;
+__device__ __forceinline__ PartWeights merge_part(float& m, float& l, float part_m, float part_l) {
+    const float next = fmaxf(m, part_m), low = fminf(m, part_m);
+    const float smaller = low == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(low - next);
+    const PartWeights w{m == next ? 1.0f : smaller, part_m == next ? 1.0f : smaller};
+    m = next;
+    l = __builtin_fmaf(w.part, part_l, w.keep * l);
+    return w;
+}
+__device__ __forceinline__ float merged(float sum, float part, PartWeights w) {
+    return __builtin_fmaf(w.part, part, w.keep * sum);
+}
+__device__ __forceinline__ float4v merged(float4v sum, float4v part, PartWeights w) {
+    return float4v{merged(sum[0], part[0], w), merged(sum[1], part[1], w), merged(sum[2], part[2], w),
+                   merged(sum[3], part[3], w)};
+}
+
 // Partial results that another workgroup of the launch reads: stores that
 // write through the XCD's L2 to the point where all XCDs agree, and loads that
 // do not take a line the L2 holds (sc1, device scope). A release of ordinary

@@ -499,22 +499,13 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
                         value[u][b] = __builtin_bit_cast(
                             float4v, __builtin_amdgcn_raw_buffer_load_b128(ro, (from * kDP + f0 + 4 * b) * 4, 0, kDeviceScope));
                 }
-                float m_next = m;
-#pragma unroll
-                for (int u = 0; u < kBatch; ++u) m_next = fmaxf(m_next, state[u][0]);
-                if (m_next == -INFINITY) continue;  // no key visible so far
-                const float rescale = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - m_next);
-                l *= rescale;
-#pragma unroll
-                for (int b = 0; b < kBlocks; ++b) acc[b] *= rescale;
-                m = m_next;
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
-                    const bool counts = s0 + u < p.splits && state[u][0] != -INFINITY;
-                    const float weight = counts ? __builtin_amdgcn_exp2f(state[u][0] - m) : 0.0f;
-                    l += weight * state[u][1];
+                    if (s0 + u < p.splits) {
+                        const PartWeights w = merge_part(m, l, state[u][0], state[u][1]);
 #pragma unroll
-                    for (int b = 0; b < kBlocks; ++b) acc[b] += weight * value[u][b];
+                        for (int b = 0; b < kBlocks; ++b) acc[b] = merged(acc[b], value[u][b], w);
+                    }
                 }
             }
         }
