@@ -1,8 +1,10 @@
 // Host-only program over the rules that the launches of the HIP library follow
-// (csrc/attention_common.h): the edges of the addressing, restated here from
-// single bytes. Prints one line per failure; exit status 1 if there was one.
+// (csrc/attention_common.h, csrc/attention_rules.h): the edges of the addressing,
+// restated here from single bytes, and calls on both sides of the dispatch rules
+// for a device of 256 compute units. Prints one line per failure; exit status 1 if there was one.
 
 #include "attention_common.h"
+#include "attention_rules.h"
 
 #include <cstdio>
 
@@ -34,9 +36,55 @@ void k8_pieces_stay_inside_the_head() {
     }
 }
 
+tilemix::AttnParams call(int heads, int M, int N, int d, bool causal) {
+    tilemix::AttnParams p{};
+    p.heads = heads;
+    p.M = M;
+    p.N = N;
+    p.d = d;
+    p.causal = causal;
+    p.q_blocks = (M - 1) / tilemix::kRowsPerGroup + 1;
+    return p;
+}
+
+// The 256-row kernel: never for heads of one 128-row block, never in more
+// rounds of workgroups than the 128-row kernel's, never for a causal walk of
+// fewer than 32 tiles however many keys there are; and the measured calls on
+// both sides of the line.
+void wide_kernel_rule() {
+    using namespace tilemix;
+    constexpr int kUnits = 256;
+    auto expect = [](int heads, int M, int N, int d, bool causal, bool wide) {
+        if (wide_pays(call(heads, M, N, d, causal), kUnits) == wide) return;
+        std::printf("wide_pays(%d heads x %d x %d x %d, causal %d) is not %d\n", heads, M, N, d, causal, wide);
+        ++failures;
+    };
+    for (int heads = 1; heads <= 2048; ++heads)
+        for (int M : {1, 16, 64, 128, 129, 256, 300, 384, 640, 1152}) {
+            const bool wide = wide_pays(call(heads, M, 4096, 128, false), kUnits);
+            const int blocks = (M + 127) / 128;
+            const int wide_rounds = (heads * ((blocks + 1) / 2) + kUnits - 1) / kUnits;
+            const int rounds = (heads * blocks + 2 * kUnits - 1) / (2 * kUnits);
+            if (wide && (blocks == 1 || wide_rounds > rounds)) expect(heads, M, 4096, 128, false, false);
+            if (M < 1920) expect(heads, M, 8192, 128, true, false);
+        }
+    expect(64, 2048, 2048, 64, false, true);
+    expect(32, 16384, 16384, 128, false, true);
+    expect(64, 4096, 4096, 128, true, true);
+    expect(64, 4096, 2048, 128, true, true);
+    expect(256, 300, 4096, 128, false, true);
+    expect(256, 129, 4096, 128, false, true);
+    expect(512, 384, 4096, 128, false, false);
+    expect(16, 2048, 2048, 64, false, false);
+    expect(48, 3000, 3000, 128, false, false);
+    expect(64, 1024, 1024, 128, false, false);
+    expect(16, 4096, 4096, 128, true, false);
+}
+
 }  // namespace
 
 int main() {
+    wide_kernel_rule();
     k8_pieces_stay_inside_the_head();
     if (failures == 0) std::printf("launch rules OK\n");
     return failures != 0;

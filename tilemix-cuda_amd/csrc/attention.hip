@@ -52,6 +52,7 @@
 //    two halves of the wave, not through LDS.
 
 #include "attention_common.h"
+#include "attention_rules.h"
 #include "tilemix_capi.h"
 
 #include <atomic>
@@ -65,13 +66,7 @@ namespace {
 
 constexpr int kThreadsPerGroup = 256;
 constexpr int kWavesPerGroup = kThreadsPerGroup / kWave;
-constexpr int kRowsPerGroup = 128;  // one Q quantization block
 constexpr int kRowsPerWave = 32;
-#ifndef TILEMIX_GROUPS_PER_CU
-#define TILEMIX_GROUPS_PER_CU 2
-#endif
-// Workgroups per CU the register allocation is sized for (launch bound).
-constexpr int kGroupsPerCU = TILEMIX_GROUPS_PER_CU;
 
 template <int DC>
 struct Layout {
@@ -1165,7 +1160,6 @@ constexpr int kWideThreads = 512;
 #define TILEMIX_INLINE __attribute__((always_inline))  // lambdas the walk uses twice
 constexpr int kWideWaves = kWideThreads / kWave;
 constexpr int kWideRows = 256;
-constexpr int kWideMaxTiles = 1024;  // key tiles that the table holds
 
 // A wave's view of one visited tile: cell bits (2 r + key half) in INT8 and
 // SKIP, what any wave of the workgroup needs of it, how this wave scores it.
@@ -1751,32 +1745,6 @@ hipError_t check_device(int* compute_units = nullptr) {
         if (compute_units) *compute_units = properties.multiProcessorCount;
     }
     return supported ? hipSuccess : hipErrorNotSupported;
-}
-
-// Whether the wide kernel is the faster one for a launch that it can take
-// (whole 16-byte pieces, head dimensions 33 .. 64 and 97 .. 128, fast P.V, no
-// split, no verification outputs). It halves the tile loads and keeps the
-// matrix cores and exponentials of a CU's two halves apart, but has one
-// workgroup per CU, whose prologue and epilogue nothing overlaps: it needs long
-// walks and whole rounds of workgroups. Rows of a reversed round keep the
-// direction that the 128-row kernel gives them (even number of row blocks).
-// 128-row kernel | wide kernel (us), 64 features: 64 heads x 2048 101.3 | 96.9;
-// 32 x 2048 routed 53.3 | 51.1; 64 x 4096 causal 191.0 | 186.8; 16 x 2048 37.5 |
-// 39.6; 64 x 1024 25.8 | 26.2. 128 features: 32 x 16384 routed 3551 | 3363; 32 x
-// 8192 three-way 847 | 815; 32 x 8192 dense 1064 | 1033, causal 557 | 541; 64 x
-// 4096 causal 320.6 | 315.7; 16 x 4096 causal 106.3 | 108.2; 48 x 3000 (2.25
-// rounds) 258.4 | 263.5; 64 x 1024 46.8 | 48.0; 16 x 2048 48.6 | 53.5. Precise
-// P.V, whose matrix slot is twice as long: 32 x 4096 causal 203.8 | 207.2.
-bool wide_pays(const AttnParams& p, int compute_units) {
-    constexpr int kLongWalk = 32;  // key tiles
-    const int tiles = (p.N - 1) / kTileKeys + 1;
-    if (compute_units <= 0 || tiles < kLongWalk || tiles > kWideMaxTiles) return false;
-    if (p.reverse_slots > 0 && p.q_blocks % 2 != 0) return false;
-    const std::int64_t workgroups = static_cast<std::int64_t>(p.heads) * ((p.q_blocks + 1) / 2);
-    if (p.causal) return workgroups >= 2 * static_cast<std::int64_t>(compute_units);
-    // Whole rounds: at most a tenth of the last one empty.
-    const std::int64_t rounds = (workgroups + compute_units - 1) / compute_units;
-    return 10 * workgroups >= 9 * rounds * compute_units;
 }
 
 // `units`: the device's compute units (check_device).

@@ -535,8 +535,9 @@ constexpr int kLongWalk = 64;  // steps of a workgroup
 // heads x 512 keys x 64: 60.9 us with eight waves, 46.7 with four). Below,
 // eight waves share a head's keys (200 heads x 4096 x 64: 33.9 us, with four
 // 36.7). With rows of more than 128 bytes that take 16-byte loads, the prefill
-// kernel's tile loads, whole KiB by each wave, read faster then (1000 heads x
-// 1024 x 128 dense: 95.6 us against 121): decode_worthwhile.
+// kernel's tile loads, whole KiB by each wave, read faster then (the 128-row one;
+// 1000 heads x 1024 x 128 dense: 95.6 us against 121; 512 heads x 16 rows x 4096 x
+// 128 dense 180 against 232, half INT8 161 against 200): decode_worthwhile.
 constexpr int kManyHeads = 512;
 
 template <int kBlocks, int kPiece, bool kPrecise, int kWaves, bool kStream>
