@@ -67,13 +67,15 @@ int tilemix_quantize_qk(const uint16_t* Q, const uint16_t* K, int8_t* Q8, int8_t
  * device array inside the library (one per GPU) and are merged into O by a
  * second kernel on `stream`. Split calls on one device are ordered through one event (each
  * waits for the previous one's merge, on any stream); a call made while
- * `stream` is being captured into a graph takes the unsplit launch.
+ * `stream` is being captured into a graph uses neither array nor event: one
+ * workgroup takes the ranges of a block in turn, and the replay equals the
+ * eager call to the bit.
  * tilemix_attention_batched splits a call of few, long row blocks (at least 16
  * key tiles) in the same way where that saves time.
  * A call of M <= 16 query rows (here and in tilemix_attention_batched without
  * a causal mask) is served by a kernel of its own, which splits the keys of
  * its heads over workgroups of the same launch through the same workspace,
- * ordered and unsplit under capture in the same way.
+ * ordered, and under capture in turn, in the same way.
  */
 int tilemix_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* V, float* O,
                       int M, int N, int d, float score_scale, void* stream,

@@ -514,10 +514,19 @@ __device__ __forceinline__ void prepare_q(const AttnParams& p, std::int64_t head
 // is read (V's reaches only features past d of O). A tile of which a piece would
 // end past the head comes in by dwords instead (load_tile_dwords). 0: single
 // elements.
-// kSplit: the workgroup covers one range of key tiles of its 128-row block
-// and writes that range's partial row state (AttnParams::splits).
-template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
+// kRange: what a workgroup covers of its 128-row block's key tiles. kWhole: all
+// of them. kSplit: one range (AttnParams::splits), whose partial row state it
+// writes. kInTurn: all ranges of a split call one after the other, each with a
+// row state of its own, merged as split_combine_kernel merges them: the split
+// call's bits without a workspace, for a stream that is being captured. It
+// holds a second O in LDS, so one workgroup per CU; a call that is split has no
+// more. Reading and writing that O takes 1.1 to 1.5 us a range: captured, 8
+// heads x 512 x 8192 x 128 take 197 us (kWhole, whose sums have another order,
+// 174), 4 x 2048 x 128 causal 56 (47), 12 x 1003 x 72 causal precise 38 (36).
+enum class KeyRange { kWhole, kSplit, kInTurn };
+template <int DC, int kPiece, bool kPrecise, bool kDots, KeyRange kRange>
 __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kernel(const AttnParams p) {
+    constexpr bool kSplit = kRange == KeyRange::kSplit, kInTurn = kRange == KeyRange::kInTurn;
     using L = Layout<DC>;
     constexpr int kDP = L::kDP;
     constexpr int kOB = DC;               // 32-feature output blocks
@@ -528,6 +537,10 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     __shared__ unsigned group_bits[kWavesPerGroup];
     // Landing area of the spare DMA slots (written with zeros, never read).
     __shared__ __attribute__((aligned(16))) unsigned char lds_spare[1024];
+    // kInTurn: the merged O. Dynamic (kMergedBytes), as with a size that it knows
+    // the compiler allocates registers for one workgroup per CU and keeps the
+    // accumulators in AGPRs, copied to and fro: 273 us for the first call above.
+    extern __shared__ float4v lds_merged[];
     unsigned char* const lds_k = smem;
     unsigned char* const lds_v = smem + L::kKBytes;
     unsigned char* const lds_k8 = smem + L::kKBytes + L::kVBytes;
@@ -578,7 +591,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     // Key tiles are visited first to last, or last to first in a reversed
     // round (AttnParams::reverse_slots; the online softmax takes the tiles in
     // any order).
-    const int step = (!kSplit && reversed_round(blockIdx.x, p.reverse_slots)) ? -1 : 1;
+    const int step = (kRange == KeyRange::kWhole && reversed_round(blockIdx.x, p.reverse_slots)) ? -1 : 1;
 
     // ------------------------------------------------------ routing masks
     // One pass decodes four tiles: lane 16t + c decodes cell c (row c / 2,
@@ -788,6 +801,39 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     for (int fb = 0; fb < kOB; ++fb) st.o[fb] = float16v{};
     st.lsum = 0.0f;
     st.m = -INFINITY;
+    // kInTurn: the merge of the ranges before the current one, which ends
+    // before tile turn_end, and how many ranges have not been merged. Its O lies
+    // in LDS, each thread's values its own.
+    float merged_m = -INFINITY, merged_l = 0.0f;
+    int turn_end = p.split_tiles, turns = p.splits;
+    if constexpr (kInTurn)
+        for (int x = 0; x < 4 * kOB; ++x) lds_merged[x * kThreadsPerGroup + tid] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+    auto end_turn = [&]() {
+        float a = st.lsum, b = st.lsum;
+        permlane32_swap(a, b);
+        const PartWeights w = merge_part(merged_m, merged_l, st.m, a + b);
+        float4v* const mine = lds_merged + tid;
+#pragma unroll
+        for (int fb = 0; fb < kOB; fb += kOB % 2 ? 1 : 2) {
+            constexpr int kBatch = kOB % 2 ? 4 : 8;
+            float4v sum[kBatch];
+#pragma unroll
+            for (int x = 0; x < kBatch; ++x) sum[x] = mine[(4 * fb + x) * kThreadsPerGroup];
+            asm volatile("" ::: "memory");  // reads first: they wait once a batch
+#pragma unroll
+            for (int x = 0; x < kBatch; ++x) {
+                const float16v& o = st.o[fb + x / 4];
+                const int e = 4 * (x % 4);
+                mine[(4 * fb + x) * kThreadsPerGroup] = merged(sum[x], float4v{o[e], o[e + 1], o[e + 2], o[e + 3]}, w);
+            }
+        }
+#pragma unroll
+        for (int fb = 0; fb < kOB; ++fb) st.o[fb] = float16v{};
+        st.lsum = 0.0f;
+        st.m = -INFINITY;
+        turn_end += p.split_tiles;
+        --turns;
+    };
     const bool positive_scale = p.score_scale >= 0.0f;
 
     const int key_tiles64 = (N - 1) / kTileKeys + 1;
@@ -844,6 +890,8 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     // the tile's loads and barriers only: its probabilities would all be 0,
     // so the softmax and P.V would leave m, l and O unchanged.
     while (in_walk(j)) {
+        if constexpr (kInTurn)
+            while (j >= turn_end) end_turn();
         const int k0 = j * kTileKeys;
         const std::uint32_t int8_mask = cur_int8, skip_mask = cur_skip;
         tile_barrier();  // K_j, V_j landed; every wave finished P.V of the previous tile
@@ -1036,6 +1084,17 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
         v_buffer ^= 1;
     }
 
+    if constexpr (kInTurn) {
+        // Ranges without a visible tile too: each is a part of the merge.
+        while (turns > 0) end_turn();
+#pragma unroll
+        for (int x = 0; x < 4 * kOB; ++x) {
+            const float4v value = lds_merged[x * kThreadsPerGroup + tid];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st.o[x / 4][4 * (x % 4) + e] = value[e];
+        }
+    }
+
     // Routing trace of tiles a causal workgroup never visits (of its range, the
     // last one's to the end).
     if (kDots && p.trace && p.causal) {
@@ -1096,7 +1155,7 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
     } else {
         float a = st.lsum, b = st.lsum;
         permlane32_swap(a, b);  // the row's other half, held by lane ^ 32
-        const float l = a + b;
+        const float l = kInTurn ? merged_l : a + b;
         const float inverse = l > 0.0f ? 1.0f / l : 0.0f;
         const int row = qw + q;
         if constexpr (kStaged) {
@@ -1648,21 +1707,24 @@ __global__ __launch_bounds__(256) void split_combine_kernel(const AttnParams p) 
     store_output(Oh, p.o_dtype, static_cast<std::int64_t>(row) * p.o_row + f0, acc * inverse, d - f0, p.o_vector != 0);
 }
 
-template <int DC, int kPiece, bool kPrecise, bool kDots, bool kSplit>
-hipError_t launch_variant(const AttnParams& p, hipStream_t stream) {
+template <int DC, int kPiece, bool kDots, KeyRange kRange>
+hipError_t launch_variant(const AttnParams& p, bool precise, hipStream_t stream) {
     const unsigned blocks = static_cast<unsigned>(p.q_blocks) * static_cast<unsigned>(p.heads) *
-                            static_cast<unsigned>(kSplit ? p.splits : 1);
-    attention_kernel<DC, kPiece, kPrecise, kDots, kSplit><<<blocks, kThreadsPerGroup, 0, stream>>>(p);
+                            static_cast<unsigned>(kRange == KeyRange::kSplit ? p.splits : 1);
+    constexpr unsigned kMergedBytes = kRange == KeyRange::kInTurn ? 4 * DC * kThreadsPerGroup * sizeof(float4v) : 0;
+    if (precise)
+        attention_kernel<DC, kPiece, true, kDots, kRange><<<blocks, kThreadsPerGroup, kMergedBytes, stream>>>(p);
+    else
+        attention_kernel<DC, kPiece, false, kDots, kRange><<<blocks, kThreadsPerGroup, kMergedBytes, stream>>>(p);
     return hipGetLastError();
 }
 
+// A split call without a workspace takes its ranges in turn.
 template <int DC, int kPiece, bool kDots>
 hipError_t launch_vp(const AttnParams& p, bool precise, hipStream_t stream) {
-    if (p.splits > 1)
-        return precise ? launch_variant<DC, kPiece, true, kDots, true>(p, stream)
-                       : launch_variant<DC, kPiece, false, kDots, true>(p, stream);
-    return precise ? launch_variant<DC, kPiece, true, kDots, false>(p, stream)
-                   : launch_variant<DC, kPiece, false, kDots, false>(p, stream);
+    if (p.splits <= 1) return launch_variant<DC, kPiece, kDots, KeyRange::kWhole>(p, precise, stream);
+    return p.part_o ? launch_variant<DC, kPiece, kDots, KeyRange::kSplit>(p, precise, stream)
+                    : launch_variant<DC, kPiece, kDots, KeyRange::kInTurn>(p, precise, stream);
 }
 
 template <int DC>
@@ -1785,7 +1847,7 @@ hipError_t launch_attention(AttnParams p, int units, bool precise, hipStream_t s
 // device are ordered through one event (each waits for the previous split
 // call's last kernel, whatever its stream), so concurrent streams never share
 // the workspace at once; calls made while their stream is being captured into
-// a graph take an unsplit launch instead.
+// a graph use neither and take the same ranges of keys in turn.
 static constexpr std::size_t kSplitScratchFloats = std::size_t{8} << 20;  // 32 MiB
 static constexpr std::size_t kSplitArrivals = 1024;
 static __device__ __align__(256) float split_scratch[kSplitScratchFloats];
@@ -1936,19 +1998,21 @@ hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
 // launch_attention, with the key range split over several workgroups per
 // 128-row block when choose_split_tiles says so: the attention kernel writes
 // each split's partial rows to the workspace, split_combine_kernel merges them
-// into O, both on `stream`.
+// into O, both on `stream`. Where the workspace is not to be used, one workgroup
+// takes a block's ranges in turn, to the same bits.
 hipError_t launch_attention_split(AttnParams p, bool precise, const SplitRule& rule, hipStream_t stream) {
     int units = 0;
     const hipError_t found = check_device(&units);
     if (found != hipSuccess) return found;
     const int split_tiles = choose_split_tiles(p, precise, units, rule);
-    const int device = split_tiles > 0 ? workspace_device(stream) : -1;
-    if (device < 0) return launch_attention(p, units, precise, stream);
+    if (split_tiles == 0) return launch_attention(p, units, precise, stream);
+    int tiles = (p.N - 1) / kTileKeys + 1;
+    if (p.causal) tiles = std::min(tiles, p.q_blocks * (kRowsPerGroup / kTileKeys));
+    p.split_tiles = split_tiles;
+    p.splits = (tiles + split_tiles - 1) / split_tiles;
+    const int device = workspace_device(stream);
+    if (device < 0) return launch_attention(p, units, precise, stream);  // the ranges in turn
     return with_workspace(device, stream, [&](float* scratch, unsigned*) {
-        int tiles = (p.N - 1) / kTileKeys + 1;
-        if (p.causal) tiles = std::min(tiles, p.q_blocks * (kRowsPerGroup / kTileKeys));
-        p.split_tiles = split_tiles;
-        p.splits = (tiles + split_tiles - 1) / split_tiles;
         p.part_o = scratch;
         p.part_ml = scratch + static_cast<std::size_t>(p.heads) * p.splits * p.M * p.d;
         const hipError_t status = launch_attention(p, units, precise, stream);
@@ -1983,7 +2047,7 @@ hipError_t launch_decode_split(AttnParams p, bool precise, hipStream_t stream) {
     if (found != hipSuccess) return found;
     const int splits = plan_decode(p, units, kSplitScratchFloats, kSplitArrivals);
     const int device = splits > 1 ? workspace_device(stream) : -1;
-    if (device < 0) return launch_decode(p, 1, precise, stream);
+    if (device < 0) return launch_decode(p, splits, precise, stream);  // the ranges in turn
     return with_workspace(device, stream, [&](float* scratch, unsigned* arrivals) {
         p.part_o = scratch;
         p.arrivals = arrivals;

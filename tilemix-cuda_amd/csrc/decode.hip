@@ -138,8 +138,11 @@ struct StepData {
 
 // kBlocks: 64-feature blocks (1: d <= 64, 2: d <= 128). kPiece: bytes of a
 // contiguous load (load_halves). kWaves: waves of a workgroup. kStream: keys
-// and values are loaded with a non-temporal hint.
-template <int kBlocks, int kPiece, bool kPrecise, int kWaves, bool kStream>
+// and values are loaded with a non-temporal hint. kInTurn: the workgroup takes
+// all of its head's ranges one after the other and merges them as the last of
+// several workgroups does: a split call's bits without a workspace, for a
+// stream that is being captured.
+template <int kBlocks, int kPiece, bool kPrecise, int kWaves, bool kStream, bool kInTurn>
 __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(const AttnParams p) {
     constexpr int kDP = 64 * kBlocks;
     constexpr int kFpl = 4 * kBlocks;  // value features per lane
@@ -154,8 +157,8 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15;  // key of a score block (A operand), query row (B operand and results)
     const int g = lane >> 4;
-    const int head32 = blockIdx.x / p.splits;
-    const int split = blockIdx.x - head32 * p.splits;
+    const int head32 = kInTurn ? blockIdx.x : blockIdx.x / p.splits;
+    const int first_split = kInTurn ? 0 : blockIdx.x - head32 * p.splits;
     const std::int64_t head = head32;
     const int M = p.M, N = p.N, d = p.d;
 
@@ -210,259 +213,283 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
         if ((skip_word >> bit) & 1u) return TILEMIX_ROUTE_SKIP;
         return ((route_word >> bit) & 1u) ? TILEMIX_ROUTE_INT8 : TILEMIX_ROUTE_FP16;
     };
-    // This workgroup's steps, dealt to its waves in turn. Every step is passed
-    // once by one wave, which writes its routing trace.
-    const int step_end = min((N - 1) / kStepKeys + 1, (split + 1) * p.split_tiles);
-    int code = TILEMIX_ROUTE_FP16;
-    auto next_step = [&](int step) {
-        for (; step < step_end; step += kWaves) {
-            code = code_of(step);
-            if (p.trace && lane == 0) p.trace[head * p.key_tiles32 + step] = static_cast<std::uint8_t>(code);
-            if (code != TILEMIX_ROUTE_SKIP) break;
-        }
-        return step;
-    };
-    auto load_step = [&](StepData<kBlocks>& data, int step, int route) {
-        const unsigned k0 = static_cast<unsigned>(step * kStepKeys);
-        if (route == TILEMIX_ROUTE_INT8) {
-            data.k_scale = k_scales[step >> 1];
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int m = 0; m < kBlocks; ++m)
-                    data.k[b][m] = load_bytes<kPiece, kAux>(rk8, (k0 + 16 * b) * d + k8_at[m], k8_valid[m]);
-        } else {
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int c = 0; c < kPieces; ++c)
-                    data.k[b][c] = load_halves<8, kPiece, kAux>(rk, (k0 + 16 * b) * k_row_bytes + k_at[c], k_valid[c]);
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            data.v[e] = load_halves<kFpl, kPiece, kAux>(rv, (k0 + 16 * (e / 4) + e % 4) * v_row_bytes + v_at, v_valid);
-    };
-
-    // The first step is fetched before Q is touched.
-    StepData<kBlocks> even, odd;
-    int step = next_step(split * p.split_tiles + wave);
-    int step_code = code;
-    if (step < step_end) load_step(even, step, step_code);
-
-    // ------------------------------------------------------------ Q
-    half8 qf[kPieces];
-#pragma unroll
-    for (int c = 0; c < kPieces; ++c) {
-        const int feature = 64 * (c / 2) + 16 * g + 8 * (c % 2);
-        const unsigned at = r < M ? static_cast<unsigned>(r * q_row_bytes + 2 * feature) : 0x80000000u;
-        qf[c] = __builtin_bit_cast(half8, load_halves<8, kPiece>(rq, at, r < M ? d - feature : 0));
-    }
-    int4v q8f[kBlocks];
-    float q_scale = 0.0f;
-    if (p.int8_operands) {
-        if (p.fuse_q_quant) {
-            // The head's M <= 16 rows are its one Q block, all in this wave:
-            // the quantizer's maximum (integer order of the sign-cleared fp16
-            // bits, NaNs passed over) and bytes.
-            unsigned top = 0;
-#pragma unroll
-            for (int c = 0; c < kPieces; ++c) {
-                const uint4v words = __builtin_bit_cast(uint4v, qf[c]);
-#pragma unroll
-                for (int w = 0; w < 4; ++w) top = max_u16x2(top, words[w] & 0x7fff7fffu);
+    // One range of steps, up to the merge of the workgroup's waves: the state and
+    // O of each thread's row of it.
+    float4v acc[kBlocks];
+    float row_m, row_l;
+    auto take_range = [&](int split) __attribute__((always_inline)) {
+        // This workgroup's steps, dealt to its waves in turn. Every step is passed
+        // once by one wave, which writes its routing trace.
+        const int step_end = min((N - 1) / kStepKeys + 1, (split + 1) * p.split_tiles);
+        int code = TILEMIX_ROUTE_FP16;
+        auto next_step = [&](int step) {
+            for (; step < step_end; step += kWaves) {
+                code = code_of(step);
+                if (p.trace && lane == 0) p.trace[head * p.key_tiles32 + step] = static_cast<std::uint8_t>(code);
+                if (code != TILEMIX_ROUTE_SKIP) break;
             }
-            unsigned bits = wave_max_bits(max(top & 0xffffu, top >> 16));
-            if (bits > 0x7c00u) {
-                unsigned clean = 0;
+            return step;
+        };
+        auto load_step = [&](StepData<kBlocks>& data, int step, int route) {
+            const unsigned k0 = static_cast<unsigned>(step * kStepKeys);
+            if (route == TILEMIX_ROUTE_INT8) {
+                data.k_scale = k_scales[step >> 1];
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int m = 0; m < kBlocks; ++m)
+                        data.k[b][m] = load_bytes<kPiece, kAux>(rk8, (k0 + 16 * b) * d + k8_at[m], k8_valid[m]);
+            } else {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int c = 0; c < kPieces; ++c)
+                        data.k[b][c] = load_halves<8, kPiece, kAux>(rk, (k0 + 16 * b) * k_row_bytes + k_at[c], k_valid[c]);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                data.v[e] = load_halves<kFpl, kPiece, kAux>(rv, (k0 + 16 * (e / 4) + e % 4) * v_row_bytes + v_at, v_valid);
+        };
+
+        // The first step is fetched before Q is touched.
+        StepData<kBlocks> even, odd;
+        int step = next_step(split * p.split_tiles + wave);
+        int step_code = code;
+        if (step < step_end) load_step(even, step, step_code);
+
+        // ------------------------------------------------------------ Q
+        half8 qf[kPieces];
+#pragma unroll
+        for (int c = 0; c < kPieces; ++c) {
+            const int feature = 64 * (c / 2) + 16 * g + 8 * (c % 2);
+            const unsigned at = r < M ? static_cast<unsigned>(r * q_row_bytes + 2 * feature) : 0x80000000u;
+            qf[c] = __builtin_bit_cast(half8, load_halves<8, kPiece>(rq, at, r < M ? d - feature : 0));
+        }
+        int4v q8f[kBlocks];
+        float q_scale = 0.0f;
+        if (p.int8_operands) {
+            if (p.fuse_q_quant) {
+                // The head's M <= 16 rows are its one Q block, all in this wave:
+                // the quantizer's maximum (integer order of the sign-cleared fp16
+                // bits, NaNs passed over) and bytes.
+                unsigned top = 0;
 #pragma unroll
                 for (int c = 0; c < kPieces; ++c) {
                     const uint4v words = __builtin_bit_cast(uint4v, qf[c]);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const unsigned hb = (words[e / 2] >> (16 * (e % 2))) & 0x7fffu;
-                        clean = hb <= 0x7c00u ? max(clean, hb) : clean;
-                    }
+                    for (int w = 0; w < 4; ++w) top = max_u16x2(top, words[w] & 0x7fff7fffu);
                 }
-                bits = wave_max_bits(clean);
-            }
-            const float scale = block_scale(half_bits_to_float(static_cast<std::uint16_t>(bits)));
-            const float recip = 1.0f / scale;
-            const _Float16 stored = static_cast<_Float16>(scale);
-            q_scale = static_cast<float>(stored);
-            const bool writer = split == 0 && wave == 0;
-            if (writer && lane == 0 && p.q_scales_out) p.q_scales_out[head] = __builtin_bit_cast(std::uint16_t, stored);
+                unsigned bits = wave_max_bits(max(top & 0xffffu, top >> 16));
+                if (bits > 0x7c00u) {
+                    unsigned clean = 0;
 #pragma unroll
-            for (int m = 0; m < kBlocks; ++m) {
+                    for (int c = 0; c < kPieces; ++c) {
+                        const uint4v words = __builtin_bit_cast(uint4v, qf[c]);
 #pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const uint4v words = __builtin_bit_cast(uint4v, qf[2 * m + half]);
-                    int b[8] = {};
-                    if (scale > 0.0f) {
-#pragma unroll
-                        for (int w = 0; w < 4; ++w) {
-                            b[2 * w] = quantize_half<0>(words[w], scale, recip);
-                            b[2 * w + 1] = quantize_half<1>(words[w], scale, recip);
+                        for (int e = 0; e < 8; ++e) {
+                            const unsigned hb = (words[e / 2] >> (16 * (e % 2))) & 0x7fffu;
+                            clean = hb <= 0x7c00u ? max(clean, hb) : clean;
                         }
                     }
-                    q8f[m][2 * half] = static_cast<int>(pack_bytes(b[0], b[1], b[2], b[3]));
-                    q8f[m][2 * half + 1] = static_cast<int>(pack_bytes(b[4], b[5], b[6], b[7]));
+                    bits = wave_max_bits(clean);
                 }
-                if (writer && p.q8_out && r < M) {
+                const float scale = block_scale(half_bits_to_float(static_cast<std::uint16_t>(bits)));
+                const float recip = 1.0f / scale;
+                const _Float16 stored = static_cast<_Float16>(scale);
+                q_scale = static_cast<float>(stored);
+                const bool writer = split == 0 && wave == 0;
+                if (writer && lane == 0 && p.q_scales_out) p.q_scales_out[head] = __builtin_bit_cast(std::uint16_t, stored);
+#pragma unroll
+                for (int m = 0; m < kBlocks; ++m) {
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {
+                        const uint4v words = __builtin_bit_cast(uint4v, qf[2 * m + half]);
+                        int b[8] = {};
+                        if (scale > 0.0f) {
+#pragma unroll
+                            for (int w = 0; w < 4; ++w) {
+                                b[2 * w] = quantize_half<0>(words[w], scale, recip);
+                                b[2 * w + 1] = quantize_half<1>(words[w], scale, recip);
+                            }
+                        }
+                        q8f[m][2 * half] = static_cast<int>(pack_bytes(b[0], b[1], b[2], b[3]));
+                        q8f[m][2 * half + 1] = static_cast<int>(pack_bytes(b[4], b[5], b[6], b[7]));
+                    }
+                    if (writer && p.q8_out && r < M) {
+                        const int feature = 64 * m + 16 * g;
+                        std::int8_t* const dst = p.q8_out + (head * M + r) * d + feature;
+                        for (int e = 0; e < 16 && feature + e < d; ++e)
+                            dst[e] = static_cast<std::int8_t>(q8f[m][e / 4] >> (8 * (e % 4)));
+                    }
+                }
+            } else {
+                q_scale = half_bits_to_float(p.q_scales[head]);
+                const Rsrc rq8 = buffer(p.Q8 + head * M * d, static_cast<std::int64_t>(M) * d);
+#pragma unroll
+                for (int m = 0; m < kBlocks; ++m) {
                     const int feature = 64 * m + 16 * g;
-                    std::int8_t* const dst = p.q8_out + (head * M + r) * d + feature;
-                    for (int e = 0; e < 16 && feature + e < d; ++e)
-                        dst[e] = static_cast<std::int8_t>(q8f[m][e / 4] >> (8 * (e % 4)));
+                    q8f[m] = __builtin_bit_cast(
+                        int4v, load_bytes<kPiece>(rq8, static_cast<unsigned>(r * d + feature), r < M ? d - feature : 0));
                 }
             }
-        } else {
-            q_scale = half_bits_to_float(p.q_scales[head]);
-            const Rsrc rq8 = buffer(p.Q8 + head * M * d, static_cast<std::int64_t>(M) * d);
-#pragma unroll
-            for (int m = 0; m < kBlocks; ++m) {
-                const int feature = 64 * m + 16 * g;
-                q8f[m] = __builtin_bit_cast(
-                    int4v, load_bytes<kPiece>(rq8, static_cast<unsigned>(r * d + feature), r < M ? d - feature : 0));
-            }
         }
-    }
 
-    // ------------------------------------------------------------ keys
-    float4v o[kFpl];  // o[f][i]: query row r, feature kFpl (4 g + i) + f
+        // ------------------------------------------------------------ keys
+        float4v o[kFpl];  // o[f][i]: query row r, feature kFpl (4 g + i) + f
 #pragma unroll
-    for (int f = 0; f < kFpl; ++f) o[f] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-    float row_max = -INFINITY, row_sum = 0.0f;  // row_sum: this lane's part
-    const bool positive_scale = p.score_scale >= 0.0f;
+        for (int f = 0; f < kFpl; ++f) o[f] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+        float row_max = -INFINITY, row_sum = 0.0f;  // row_sum: this lane's part
+        const bool positive_scale = p.score_scale >= 0.0f;
 
-    auto compute = [&](const StepData<kBlocks>& data, int at, int route) {
-        const int k0 = at * kStepKeys;
-        float4v s[2];  // s[b][i]: row r against key k0 + 16 b + 4 g + i
-        float c;       // log2-domain factor
-        if (route == TILEMIX_ROUTE_INT8) {
-            c = ((q_scale * half_bits_to_float(data.k_scale)) * p.score_scale) * kLog2e;
+        auto compute = [&](const StepData<kBlocks>& data, int at, int route) {
+            const int k0 = at * kStepKeys;
+            float4v s[2];  // s[b][i]: row r against key k0 + 16 b + 4 g + i
+            float c;       // log2-domain factor
+            if (route == TILEMIX_ROUTE_INT8) {
+                c = ((q_scale * half_bits_to_float(data.k_scale)) * p.score_scale) * kLog2e;
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                int4v acc{0, 0, 0, 0};
+                for (int b = 0; b < 2; ++b) {
+                    int4v acc{0, 0, 0, 0};
 #pragma unroll
-                for (int m = 0; m < kBlocks; ++m)
-                    acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(int4v, data.k[b][m]), q8f[m], acc, 0, 0, 0);
-                if (p.dots && r < M) {  // raw int32 dots (verification output)
-                    std::int32_t* const row = p.dots + (head * M + r) * static_cast<std::int64_t>(N);
+                    for (int m = 0; m < kBlocks; ++m)
+                        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(int4v, data.k[b][m]), q8f[m], acc, 0, 0, 0);
+                    if (p.dots && r < M) {  // raw int32 dots (verification output)
+                        std::int32_t* const row = p.dots + (head * M + r) * static_cast<std::int64_t>(N);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (k0 + 16 * b + 4 * g + i < N) row[k0 + 16 * b + 4 * g + i] = acc[i];
+                        for (int i = 0; i < 4; ++i)
+                            if (k0 + 16 * b + 4 * g + i < N) row[k0 + 16 * b + 4 * g + i] = acc[i];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[b][i] = static_cast<float>(acc[i]);
                 }
+            } else {
+                c = p.score_log2;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) s[b][i] = static_cast<float>(acc[i]);
-            }
-        } else {
-            c = p.score_log2;
+                for (int b = 0; b < 2; ++b) {
+                    s[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                s[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int m = 0; m < kPieces; ++m)
-                    s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, data.k[b][m]), qf[m], s[b], 0, 0, 0);
-            }
-        }
-        const bool tail = k0 + kStepKeys > N;
-        if (tail || !positive_scale) {  // explicit scores
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    s[b][i] *= c;
-                    if (k0 + 16 * b + 4 * g + i >= N) s[b][i] = -INFINITY;
+                    for (int m = 0; m < kPieces; ++m)
+                        s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, data.k[b][m]), qf[m], s[b], 0, 0, 0);
                 }
-            c = 1.0f;
+            }
+            const bool tail = k0 + kStepKeys > N;
+            if (tail || !positive_scale) {  // explicit scores
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        s[b][i] *= c;
+                        if (k0 + 16 * b + 4 * g + i >= N) s[b][i] = -INFINITY;
+                    }
+                c = 1.0f;
+            }
+            const float top = max3(max3(s[0][0], s[0][1], s[0][2]), max3(s[0][3], s[1][0], s[1][1]),
+                                   max3(s[1][2], s[1][3], s[1][3])) * c;  // c >= 0
+            if (__any(top > row_max + kLazyRescale)) {
+                const float m_new = fmaxf(row_max, groups_max(top));
+                const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(row_max - m_new);
+                row_max = m_new;
+#pragma unroll
+                for (int f = 0; f < kFpl; ++f) o[f] *= alpha;
+                row_sum *= alpha;
+            }
+            const float neg_m = row_max == -INFINITY ? 0.0f : -row_max;
+            half8 ph, pl;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e / 4][e % 4], c, neg_m));
+                const _Float16 hv = static_cast<_Float16>(v);
+                ph[e] = hv;
+                if constexpr (kPrecise) pl[e] = static_cast<_Float16>(v - static_cast<float>(hv));
+            }
+            const half2v ones{1.0f16, 1.0f16};
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                row_sum = __builtin_amdgcn_fdot2(half2v{ph[e], ph[e + 1]}, ones, row_sum, false);
+                if constexpr (kPrecise) row_sum = __builtin_amdgcn_fdot2(half2v{pl[e], pl[e + 1]}, ones, row_sum, false);
+            }
+#pragma unroll
+            for (int f = 0; f < kFpl; ++f) {
+                // Keys of slots 2t, 2t + 1 for feature f of this lane's kFpl.
+                constexpr unsigned kLow = 0x05040100u, kHigh = 0x07060302u;
+                uint4v a;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    a[t] = __builtin_amdgcn_perm(data.v[2 * t + 1][f / 2], data.v[2 * t][f / 2], f % 2 ? kHigh : kLow);
+                o[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), ph, o[f], 0, 0, 0);
+                if constexpr (kPrecise)
+                    o[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), pl, o[f], 0, 0, 0);
+            }
+        };
+
+        // Two steps per iteration, each fetching the other's data before it
+        // computes its own; every wave leaves when its steps run out.
+        while (step < step_end) {
+            const int second = next_step(step + kWaves);
+            const int second_code = code;
+            if (second < step_end) load_step(odd, second, second_code);
+            compute(even, step, step_code);
+            if (second >= step_end) break;
+            step = next_step(second + kWaves);
+            step_code = code;
+            if (step < step_end) load_step(even, step, step_code);
+            compute(odd, second, second_code);
         }
-        const float top = max3(max3(s[0][0], s[0][1], s[0][2]), max3(s[0][3], s[1][0], s[1][1]),
-                               max3(s[1][2], s[1][3], s[1][3])) * c;  // c >= 0
-        if (__any(top > row_max + kLazyRescale)) {
-            const float m_new = fmaxf(row_max, groups_max(top));
-            const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(row_max - m_new);
-            row_max = m_new;
-#pragma unroll
-            for (int f = 0; f < kFpl; ++f) o[f] *= alpha;
-            row_sum *= alpha;
-        }
-        const float neg_m = row_max == -INFINITY ? 0.0f : -row_max;
-        half8 ph, pl;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float v = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e / 4][e % 4], c, neg_m));
-            const _Float16 hv = static_cast<_Float16>(v);
-            ph[e] = hv;
-            if constexpr (kPrecise) pl[e] = static_cast<_Float16>(v - static_cast<float>(hv));
-        }
-        const half2v ones{1.0f16, 1.0f16};
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-            row_sum = __builtin_amdgcn_fdot2(half2v{ph[e], ph[e + 1]}, ones, row_sum, false);
-            if constexpr (kPrecise) row_sum = __builtin_amdgcn_fdot2(half2v{pl[e], pl[e + 1]}, ones, row_sum, false);
+
+        // ------------------------------------------------------- merge of waves
+        const float l_row = groups_sum(row_sum);
+        if (g == 0) {
+            lds_ml[wave][r][0] = row_max;
+            lds_ml[wave][r][1] = l_row;
         }
 #pragma unroll
-        for (int f = 0; f < kFpl; ++f) {
-            // Keys of slots 2t, 2t + 1 for feature f of this lane's kFpl.
-            constexpr unsigned kLow = 0x05040100u, kHigh = 0x07060302u;
-            uint4v a;
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-                a[t] = __builtin_amdgcn_perm(data.v[2 * t + 1][f / 2], data.v[2 * t][f / 2], f % 2 ? kHigh : kLow);
-            o[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), ph, o[f], 0, 0, 0);
-            if constexpr (kPrecise)
-                o[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), pl, o[f], 0, 0, 0);
+            for (int f = 0; f < kFpl; f += 4)
+                *reinterpret_cast<float4v*>(&lds_o[wave][r][kFpl * (4 * g + i) + f]) =
+                    float4v{o[f][i], o[f + 1][i], o[f + 2][i], o[f + 3][i]};
+        __syncthreads();
+
+        const int row = min(tid >> 4, 15), f0 = kFpl * (tid & 15);
+        row_m = -INFINITY;
+        row_l = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) row_m = fmaxf(row_m, lds_ml[w][row][0]);
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) acc[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const float m_w = lds_ml[w][row][0];
+            const float weight = m_w == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_w - row_m);
+            row_l += weight * lds_ml[w][row][1];
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) acc[b] += weight * *reinterpret_cast<const float4v*>(&lds_o[w][row][f0 + 4 * b]);
         }
     };
-
-    // Two steps per iteration, each fetching the other's data before it
-    // computes its own; every wave leaves when its steps run out.
-    while (step < step_end) {
-        const int second = next_step(step + kWaves);
-        const int second_code = code;
-        if (second < step_end) load_step(odd, second, second_code);
-        compute(even, step, step_code);
-        if (second >= step_end) break;
-        step = next_step(second + kWaves);
-        step_code = code;
-        if (step < step_end) load_step(even, step, step_code);
-        compute(odd, second, second_code);
+    if constexpr (kInTurn) {
+        float4v sum[kBlocks] = {};
+        float m = -INFINITY, l = 0.0f;
+        for (int split = 0; split < p.splits; ++split) {
+            take_range(split);
+            const PartWeights w = merge_part(m, l, row_m, row_l);
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) sum[b] = merged(sum[b], acc[b], w);
+            __syncthreads();  // lds_o and lds_ml are read: the next range may write them
+        }
+        row_l = l;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) acc[b] = sum[b];
+    } else {
+        take_range(first_split);
     }
 
-    // ------------------------------------------------------- merge of waves
-    const float l_row = groups_sum(row_sum);
-    if (g == 0) {
-        lds_ml[wave][r][0] = row_max;
-        lds_ml[wave][r][1] = l_row;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int f = 0; f < kFpl; f += 4)
-            *reinterpret_cast<float4v*>(&lds_o[wave][r][kFpl * (4 * g + i) + f]) =
-                float4v{o[f][i], o[f + 1][i], o[f + 2][i], o[f + 3][i]};
-    __syncthreads();
-
-    // Thread (row, part): kFpl features of one row; rows past M - 1 (threads
-    // of the upper waves among them) only arrive.
+    // Thread (row, f0) of the merges: kFpl features of one row; rows past M - 1
+    // (threads of the upper waves among them) only arrive.
     const int row = min(tid >> 4, 15), f0 = kFpl * (tid & 15);
     const bool mine = (tid >> 4) < M;
-    float4v acc[kBlocks];
-    float m = -INFINITY, l = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) m = fmaxf(m, lds_ml[w][row][0]);
-#pragma unroll
-    for (int b = 0; b < kBlocks; ++b) acc[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-        const float m_w = lds_ml[w][row][0];
-        const float weight = m_w == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_w - m);
-        l += weight * lds_ml[w][row][1];
-#pragma unroll
-        for (int b = 0; b < kBlocks; ++b) acc[b] += weight * *reinterpret_cast<const float4v*>(&lds_o[w][row][f0 + 4 * b]);
-    }
-
     // ------------------------------------------------------ merge of splits
-    if (p.splits > 1) {
+    if (!kInTurn && p.splits > 1) {
+        const int split = first_split;
         // part_o [heads][splits][M][kDP], part_ml [heads][splits][M][2]; both
         // within the workspace, so byte offsets fit 32 bits.
         const int parts = p.heads * p.splits * M;
@@ -475,14 +502,14 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, acc[b]), ro, (part * kDP + f0 + 4 * b) * 4,
                                                        0, kDeviceScope);
             if (f0 == 0)
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, float2v{m, l}), rml, part * 8, 0,
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2v, float2v{row_m, row_l}), rml, part * 8, 0,
                                                       kDeviceScope);
         }
         if (!last_arrival(p.arrivals + head, p.splits, &lds_last)) return;
         if (mine) {
             const int first = head32 * p.splits * M + row;
-            m = -INFINITY;
-            l = 0.0f;
+            row_m = -INFINITY;
+            row_l = 0.0f;
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) acc[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
             // Batches of splits, every load of a batch issued before any use.
@@ -502,7 +529,7 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
                     if (s0 + u < p.splits) {
-                        const PartWeights w = merge_part(m, l, state[u][0], state[u][1]);
+                        const PartWeights w = merge_part(row_m, row_l, state[u][0], state[u][1]);
 #pragma unroll
                         for (int b = 0; b < kBlocks; ++b) acc[b] = merged(acc[b], value[u][b], w);
                     }
@@ -511,7 +538,7 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
         }
     }
     if (mine) {
-        const float inverse = l > 0.0f ? 1.0f / l : 0.0f;
+        const float inverse = row_l > 0.0f ? 1.0f / row_l : 0.0f;
         unsigned char* const Oh = static_cast<unsigned char*>(p.O) + head * p.o_stride * (p.o_dtype == TILEMIX_DTYPE_F32 ? 4 : 2);
         const std::int64_t at = static_cast<std::int64_t>(row) * p.o_row + f0;
 #pragma unroll
@@ -540,14 +567,20 @@ constexpr int kLongWalk = 64;  // steps of a workgroup
 // 128 dense 180 against 232, half INT8 161 against 200): decode_worthwhile.
 constexpr int kManyHeads = 512;
 
+// A split call without a workspace takes its ranges in turn.
 template <int kBlocks, int kPiece, bool kPrecise, int kWaves, bool kStream>
 void launch_decode_kernel(const AttnParams& p, hipStream_t stream) {
-    const unsigned blocks = static_cast<unsigned>(p.heads) * static_cast<unsigned>(p.splits);
-    decode_kernel<kBlocks, kPiece, kPrecise, kWaves, kStream><<<blocks, kWaves * kWave, 0, stream>>>(p);
+    const unsigned heads = static_cast<unsigned>(p.heads);
+    if (p.splits > 1 && !p.part_o)
+        decode_kernel<kBlocks, kPiece, kPrecise, kWaves, false, true><<<heads, kWaves * kWave, 0, stream>>>(p);
+    else
+        decode_kernel<kBlocks, kPiece, kPrecise, kWaves, kStream, false>
+            <<<heads * static_cast<unsigned>(p.splits), kWaves * kWave, 0, stream>>>(p);
 }
 
-// The number of waves (which orders a row's sums) depends on sizes only, never
-// on alignment or routes.
+// The number of waves, which orders a row's sums as the split does, depends on
+// sizes and the device's compute units (through split_tiles) only: never on
+// alignment or routes, nor on whether the stream is being captured.
 template <int kBlocks, int kPiece, bool kPrecise>
 void launch_decode_variant(const AttnParams& p, hipStream_t stream) {
     const bool large = static_cast<std::int64_t>(p.heads) * p.N * p.d * 4 > kStreamBytes;
