@@ -1693,14 +1693,12 @@ __global__ __launch_bounds__(256) void split_combine_kernel(const AttnParams p) 
                 for (int e = 0; e < 4; ++e) value[b][e] = f0 + e < d ? src[e] : 0.0f;
             }
         }
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-            if (s0 + b < splits) {
-                const bool there = state[b][1] != kNoPart;
-                const PartWeights w = merge_part(m, l, there ? state[b][0] : -INFINITY, there ? state[b][1] : 0.0f);
-                acc = merged(acc, there ? value[b] : float4v{0.0f, 0.0f, 0.0f, 0.0f}, w);
-            }
-        }
+        merge_batch<kBatch, false>(
+            m, l, splits - s0,
+            [&](int b) TILEMIX_INLINE { return state[b][1] != kNoPart ? state[b] : float2v{-INFINITY, 0.0f}; },
+            [&](int b, PartWeights w) TILEMIX_INLINE {
+                acc = merged(acc, state[b][1] != kNoPart ? value[b] : float4v{0.0f, 0.0f, 0.0f, 0.0f}, w);
+            });
     }
     const float inverse = l > 0.0f ? 1.0f / l : 0.0f;
     unsigned char* const Oh = static_cast<unsigned char*>(p.O) + head * p.o_stride * (p.o_dtype == TILEMIX_DTYPE_F32 ? 4 : 2);

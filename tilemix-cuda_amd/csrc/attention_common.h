@@ -278,6 +278,47 @@ __device__ __forceinline__ float4v merged(float4v sum, float4v part, PartWeights
                    merged(sum[3], part[3], w)};
 }
 
+// merge_part of the states state(b), b = 0 .. min(count, kBatch) - 1, in order;
+// add(b, w) is to take part b's O in. Whole groups of four go without a branch
+// between, so that their exponentials overlap. kMany: groups in which no part
+// raises the maximum leave out the factor, 1 then, of what is merged so far: the
+// same bits in half of the instructions, which pays for many parts and O values
+// a thread (a decode head of 256 parts: 62 us with a branch a part, 58.5 in
+// groups, 54.2 so), not in the combine (12 heads x 1003 x 72 causal precise, 16
+// parts: 24.2 us in groups, 24.9 so).
+template <int kBatch, bool kMany, typename State, typename Add>
+__device__ __forceinline__ void merge_batch(float& m, float& l, int count, State&& state, Add&& add) {
+    auto general = [&](int b) __attribute__((always_inline)) {
+        const float2v s = state(b);
+        const PartWeights w = merge_part(m, l, s[0], s[1]);
+        add(b, w);
+    };
+#pragma unroll
+    for (int group = 0; group < kBatch; group += 4) {
+        if (group + 4 <= count) {
+            float top = -INFINITY;
+#pragma unroll
+            for (int b = group; b < group + 4; ++b) top = fmaxf(top, state(b)[0]);
+            if (kMany && __all(top <= m && m != -INFINITY)) {
+#pragma unroll
+                for (int b = group; b < group + 4; ++b) {
+                    const float2v s = state(b);
+                    const PartWeights w{1.0f, s[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s[0] - m)};
+                    l = __builtin_fmaf(w.part, s[1], l);
+                    add(b, w);
+                }
+            } else {
+#pragma unroll
+                for (int b = group; b < group + 4; ++b) general(b);
+            }
+        } else {
+#pragma unroll
+            for (int b = group; b < group + 4; ++b)
+                if (b < count) general(b);
+        }
+    }
+}
+
 // Partial results that another workgroup of the launch reads: stores that
 // write through the XCD's L2 to the point where all XCDs agree, and loads that
 // do not take a line the L2 holds (sc1, device scope). A release of ordinary

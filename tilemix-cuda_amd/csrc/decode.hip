@@ -39,6 +39,7 @@
 #include "tilemix_capi.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace tilemix {
 namespace {
@@ -513,28 +514,32 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void decode_kernel(cons
 #pragma unroll
             for (int b = 0; b < kBlocks; ++b) acc[b] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
             // Batches of splits, every load of a batch issued before any use.
-            constexpr int kBatch = 8;
-            for (int s0 = 0; s0 < p.splits; s0 += kBatch) {
-                float2v state[kBatch];
-                float4v value[kBatch][kBlocks];
+            auto merge_parts = [&](auto batch) __attribute__((always_inline)) {
+                constexpr int kBatch = decltype(batch)::value;
+                for (int s0 = 0; s0 < p.splits; s0 += kBatch) {
+                    float2v state[kBatch];
+                    float4v value[kBatch][kBlocks];
 #pragma unroll
-                for (int u = 0; u < kBatch; ++u) {
-                    const int from = first + min(s0 + u, p.splits - 1) * M;
-                    state[u] = __builtin_bit_cast(float2v, __builtin_amdgcn_raw_buffer_load_b64(rml, from * 8, 0, kDeviceScope));
+                    for (int u = 0; u < kBatch; ++u) {
+                        const int from = first + min(s0 + u, p.splits - 1) * M;
+                        state[u] = __builtin_bit_cast(float2v, __builtin_amdgcn_raw_buffer_load_b64(rml, from * 8, 0, kDeviceScope));
 #pragma unroll
-                    for (int b = 0; b < kBlocks; ++b)
-                        value[u][b] = __builtin_bit_cast(
-                            float4v, __builtin_amdgcn_raw_buffer_load_b128(ro, (from * kDP + f0 + 4 * b) * 4, 0, kDeviceScope));
-                }
-#pragma unroll
-                for (int u = 0; u < kBatch; ++u) {
-                    if (s0 + u < p.splits) {
-                        const PartWeights w = merge_part(row_m, row_l, state[u][0], state[u][1]);
-#pragma unroll
-                        for (int b = 0; b < kBlocks; ++b) acc[b] = merged(acc[b], value[u][b], w);
+                        for (int b = 0; b < kBlocks; ++b)
+                            value[u][b] = __builtin_bit_cast(
+                                float4v, __builtin_amdgcn_raw_buffer_load_b128(ro, (from * kDP + f0 + 4 * b) * 4, 0, kDeviceScope));
                     }
+                    merge_batch<kBatch, true>(
+                        row_m, row_l, p.splits - s0, [&](int u) __attribute__((always_inline)) { return state[u]; },
+                        [&](int u, PartWeights w) __attribute__((always_inline)) {
+#pragma unroll
+                            for (int b = 0; b < kBlocks; ++b) acc[b] = merged(acc[b], value[u][b], w);
+                        });
                 }
-            }
+            };
+            if (p.splits <= 8)
+                merge_parts(std::integral_constant<int, 8>{});
+            else
+                merge_parts(std::integral_constant<int, 16>{});
         }
     }
     if (mine) {
