@@ -81,10 +81,39 @@ void wide_kernel_rule() {
     expect(16, 4096, 4096, 128, true, false);
 }
 
+// The decode kernel: up to one head per CU, and beyond that for rows of at most
+// 128 bytes or rows that only single elements can read.
+void decode_rule() {
+    using namespace tilemix;
+    auto expect = [](int heads, int d, std::int64_t k_row, bool decode) {
+        AttnParams p = call(heads, 4, 2048, d, false);
+        p.q_row = p.v_row = d;
+        p.k_row = k_row;
+        p.q_stride = 4 * d;
+        p.k_stride = 2048 * k_row;
+        p.v_stride = 2048 * d;
+        if (decode_worthwhile(p, 256) == decode) return;
+        std::printf("decode_worthwhile(%d heads, d %d, row %d) is not %d\n", heads, d, static_cast<int>(k_row), decode);
+        ++failures;
+    };
+    for (int d : {128, 112, 100, 72}) {
+        expect(1, d, d, true);
+        expect(256, d, d, true);
+        expect(257, d, d, false);
+        expect(511, d, d, false);
+        expect(2000, d, d, false);
+        expect(300, d, d + 2, false);
+        expect(300, d, d + 1, true);
+    }
+    for (int d : {64, 40, 33}) expect(300, d, d, true);
+    for (int d : {65, 102}) expect(1000, d, d, true);
+}
+
 }  // namespace
 
 int main() {
     wide_kernel_rule();
+    decode_rule();
     k8_pieces_stay_inside_the_head();
     if (failures == 0) std::printf("launch rules OK\n");
     return failures != 0;

@@ -1998,10 +1998,7 @@ hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
 // each split's partial rows to the workspace, split_combine_kernel merges them
 // into O, both on `stream`. Where the workspace is not to be used, one workgroup
 // takes a block's ranges in turn, to the same bits.
-hipError_t launch_attention_split(AttnParams p, bool precise, const SplitRule& rule, hipStream_t stream) {
-    int units = 0;
-    const hipError_t found = check_device(&units);
-    if (found != hipSuccess) return found;
+hipError_t launch_attention_split(AttnParams p, int units, bool precise, const SplitRule& rule, hipStream_t stream) {
     const int split_tiles = choose_split_tiles(p, precise, units, rule);
     if (split_tiles == 0) return launch_attention(p, units, precise, stream);
     int tiles = (p.N - 1) / kTileKeys + 1;
@@ -2032,17 +2029,14 @@ hipError_t launch_attention_split(AttnParams p, bool precise, const SplitRule& r
 // four. Measured against it, 128 features: 4 heads x 64 keys 9.5 us either
 // way; 32 x 1024 30.1 -> 12.7 us; 32 x 16384 428 -> 54 us. Verification
 // outputs do not change the choice, so they never change O.
-bool decode_ok(const AttnParams& p) {
+bool decode_ok(const AttnParams& p, int units) {
     constexpr std::int64_t kReach = std::int64_t{1} << 30;  // halves
     return p.M <= kMaxDecodeRows && !p.causal && p.q_row * kMaxDecodeRows < kReach &&
            (p.N + std::int64_t{64}) * p.k_row < kReach && (p.N + std::int64_t{64}) * p.v_row < kReach &&
-           decode_worthwhile(p);
+           decode_worthwhile(p, units);
 }
 
-hipError_t launch_decode_split(AttnParams p, bool precise, hipStream_t stream) {
-    int units = 0;
-    const hipError_t found = check_device(&units);
-    if (found != hipSuccess) return found;
+hipError_t launch_decode_split(AttnParams p, int units, bool precise, hipStream_t stream) {
     const int splits = plan_decode(p, units, kSplitScratchFloats, kSplitArrivals);
     const int device = splits > 1 ? workspace_device(stream) : -1;
     if (device < 0) return launch_decode(p, splits, precise, stream);  // the ranges in turn
@@ -2051,6 +2045,15 @@ hipError_t launch_decode_split(AttnParams p, bool precise, hipStream_t stream) {
         p.arrivals = arrivals;
         return launch_decode(p, splits, precise, stream);
     });
+}
+
+// The kernel that takes the call.
+hipError_t launch_call(const AttnParams& p, bool precise, const SplitRule& rule, hipStream_t stream) {
+    int units = 0;
+    const hipError_t found = check_device(&units);
+    if (found != hipSuccess) return found;
+    return decode_ok(p, units) ? launch_decode_split(p, units, precise, stream)
+                               : launch_attention_split(p, units, precise, rule, stream);
 }
 
 // O takes whole vector stores: 16-byte fp32 or 8-byte 16-bit pieces of rows.
@@ -2123,8 +2126,7 @@ extern "C" int tilemix_attention(const std::uint16_t* Q, const std::uint16_t* K,
     // suite checks 1e-5 + 1e-4|x| against fp64), so P.V runs in split precision.
     // A head too small to fill the device has its key range split.
     p.o_vector = o_vector(p);
-    if (decode_ok(p)) return launch_decode_split(p, /*precise=*/true, static_cast<hipStream_t>(stream));
-    return launch_attention_split(p, /*precise=*/true, kSplitHead, static_cast<hipStream_t>(stream));
+    return launch_call(p, /*precise=*/true, kSplitHead, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tilemix_attention_batched(const TileMixBatchedArgs* args, void* stream) {
@@ -2199,8 +2201,7 @@ extern "C" int tilemix_attention_batched(const TileMixBatchedArgs* args, void* s
         p.q_scales_out = a.q_scales;
     }
     p.o_vector = o_vector(p);
-    if (decode_ok(p)) return launch_decode_split(p, a.precise != 0, static_cast<hipStream_t>(stream));
-    return launch_attention_split(p, a.precise != 0, kSplitBatch, static_cast<hipStream_t>(stream));
+    return launch_call(p, a.precise != 0, kSplitBatch, static_cast<hipStream_t>(stream));
 }
 
 extern "C" std::size_t tilemix_routing_words_per_row_c(int N, int key_tiles_per_group) {

@@ -418,12 +418,11 @@ __host__ __device__ constexpr bool k8_pieces_pass_end(int k0, int N, int d) {
     return last_row * d + (d + 15) / 16 * 16 > static_cast<std::int64_t>(N) * d;
 }
 
-// decode.hip: M <= kMaxDecodeRows query rows per head. decode_worthwhile:
-// whether it is the faster kernel for the call; plan_decode: workgroups
-// per head for a workspace of scratch_floats and max_arrivals counters (1:
-// none needed); launch_decode with p.part_o and p.arrivals set if splits > 1.
+// decode.hip: M <= kMaxDecodeRows query rows per head. plan_decode: workgroups
+// per head for a workspace of scratch_floats and max_arrivals counters (1: none
+// needed); launch_decode with p.part_o and p.arrivals set if splits > 1, or
+// without for the ranges in turn.
 inline constexpr int kMaxDecodeRows = 16;
-bool decode_worthwhile(const AttnParams& p);
 int plan_decode(const AttnParams& p, int compute_units, std::size_t scratch_floats, std::size_t max_arrivals);
 hipError_t launch_decode(AttnParams p, int splits, bool precise, hipStream_t stream);
 

@@ -57,4 +57,19 @@ inline bool wide_pays(const AttnParams& p, int compute_units) {
     return rounds <= narrow_rounds && 10 * workgroups >= 9 * rounds * compute_units;
 }
 
+// Whether the decode kernel is the faster one for a call that it can take. It
+// has one workgroup of eight waves per CU (four from 512 heads on), so past one
+// head per CU a second round begins; with rows of more than 128 bytes the
+// prefill kernel, whose tile loads take whole KiB by each wave and which runs
+// two heads per CU, is then the faster one if they move in pieces at all.
+// Decode | prefill (us, 4 rows a head): 256 heads x 2048 x 128 56.7 | 72.5; 260
+// 78.9 | 70.3; 300 82.4 | 72.3, half INT8 75.6 | 72.7; 480 111 | 91, half INT8 96 |
+// 82; 480 x 8192 424 | 342; 300 x 2048 x 100 130 | 90; 1000 x 1024 x 72 76 | 67;
+// rows at 4-byte addresses, 300 x 2048 x 128 188 | 100. Up to 64 features: 300 x
+// 2048 x 64 36.9 | 50.5, 1000 81 | 106; element by element: 300 x 1000 x 102 151 |
+// 370.
+inline bool decode_worthwhile(const AttnParams& p, int compute_units) {
+    return compute_units <= 0 || p.heads <= compute_units || p.d <= 64 || access_piece(p) == 0;
+}
+
 }  // namespace tilemix

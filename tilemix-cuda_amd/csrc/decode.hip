@@ -566,10 +566,7 @@ constexpr int kLongWalk = 64;  // steps of a workgroup
 // workgroups of four waves per CU, whose beginnings and ends overlap (2000
 // heads x 512 keys x 64: 60.9 us with eight waves, 46.7 with four). Below,
 // eight waves share a head's keys (200 heads x 4096 x 64: 33.9 us, with four
-// 36.7). With rows of more than 128 bytes that take 16-byte loads, the prefill
-// kernel's tile loads, whole KiB by each wave, read faster then (the 128-row one;
-// 1000 heads x 1024 x 128 dense: 95.6 us against 121; 512 heads x 16 rows x 4096 x
-// 128 dense 180 against 232, half INT8 161 against 200): decode_worthwhile.
+// 36.7).
 constexpr int kManyHeads = 512;
 
 // A split call without a workspace takes its ranges in turn.
@@ -619,8 +616,6 @@ void launch_decode_blocks(const AttnParams& p, bool precise, hipStream_t stream)
 // A workgroup covers at least this many steps, one for each of its waves (32
 // heads x 1024 keys x 128: 14.7 us per call with 8, 16.9 with 16).
 constexpr int kMinDecodeSteps = 8;
-
-bool decode_worthwhile(const AttnParams& p) { return p.heads < kManyHeads || p.d <= 64 || p.d % 16 != 0; }
 
 int plan_decode(const AttnParams& p, int compute_units, std::size_t scratch_floats, std::size_t max_arrivals) {
     const int steps = (p.N - 1) / kStepKeys + 1;
