@@ -10,8 +10,8 @@
  *   - every pointer is a device pointer owned by the caller; the library
  *     allocates no device memory and keeps no state between calls besides
  *     a cached per-device capability check, the fixed scratch array of
- *     tilemix_tiles_importance_noalloc, and the fixed split workspace and
- *     one ordering event per device of the attention calls (see
+ *     tilemix_tiles_importance_noalloc, and the four fixed split workspaces
+ *     per device of the attention calls, each with an ordering event (see
  *     tilemix_attention);
  *   - `stream` is a `hipStream_t` (NULL = the default stream); all work is
  *     enqueued on it and nothing synchronises;
@@ -64,9 +64,11 @@ int tilemix_quantize_qk(const uint16_t* Q, const uint16_t* K, int8_t* Q8, int8_t
  * A head too small to fill the device (its 128-row blocks under half of the
  * workgroup slots) with at least 8 key tiles of 64 has its key range split
  * over several workgroups per block, whose partial rows go to a fixed 32 MiB
- * device array inside the library (one per GPU) and are merged into O by a
- * second kernel on `stream`. Split calls on one device are ordered through one event (each
- * waits for the previous one's merge, on any stream); a call made while
+ * device array inside the library (four per GPU) and are merged into O by a
+ * second kernel on `stream`. Split calls that use the same array are ordered
+ * through its event (each waits for the previous one's merge): those of up to
+ * four streams do not wait for one another, a further stream's wait for the
+ * stream that used its array last. A call made while
  * `stream` is being captured into a graph uses neither array nor event: one
  * workgroup takes the ranges of a block in turn, and the replay equals the
  * eager call to the bit.

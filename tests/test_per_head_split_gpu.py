@@ -4,8 +4,8 @@ a range of key tiles, partial row states merged by a combine kernel through the
 library's fixed device workspace).
 
 * Calls alternating between two streams with no synchronisation in between
-  share the workspace only one at a time (the library orders split calls on a
-  device through one event): every head equals the fp64 TileMix oracle.
+  never share a workspace at once (each stream has its own, or waits for its
+  event): every head equals the fp64 TileMix oracle.
 * Ragged shapes and both O alignments (vector / element-wise combine) against
   the oracle, with the routing trace and INT32 dots exact; two of them have
   more splits than the combine takes in one batch (64 and 47).

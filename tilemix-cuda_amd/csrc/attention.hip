@@ -1839,17 +1839,21 @@ hipError_t launch_attention(AttnParams p, int units, bool precise, hipStream_t s
 }  // namespace
 }  // namespace tilemix
 
-// Workspace of the key-range splits (partial O rows and row states of every
-// split) and the arrival counters of the decode kernel. One copy per GPU, held
-// until the process ends; the library allocates nothing. Split calls on a
-// device are ordered through one event (each waits for the previous split
-// call's last kernel, whatever its stream), so concurrent streams never share
-// the workspace at once; calls made while their stream is being captured into
-// a graph use neither and take the same ranges of keys in turn.
-static constexpr std::size_t kSplitScratchFloats = std::size_t{8} << 20;  // 32 MiB
+// Workspaces of the key-range splits (partial O rows and row states of every
+// split) and the arrival counters of the decode kernel. kWorkspaces copies per
+// GPU, held until the process ends; the library allocates nothing. A stream's
+// calls use the copy that its last call used; another stream takes the one that
+// was used least recently. Calls that use the same copy are ordered through its
+// event (each waits for the previous one's last kernel, whatever its stream), so
+// concurrent streams never share a copy at once, and up to kWorkspaces of them
+// do not wait for one another (with one copy, a split call waited for all that
+// any stream had queued before its last one). Calls made while their stream is
+// being captured into a graph use none and take the same ranges of keys in turn.
+static constexpr int kWorkspaces = 4;  // as many as hardware queues, HIP's default
+static constexpr std::size_t kSplitScratchFloats = std::size_t{8} << 20;  // 32 MiB each
 static constexpr std::size_t kSplitArrivals = 1024;
-static __device__ __align__(256) float split_scratch[kSplitScratchFloats];
-static __device__ unsigned split_arrivals[kSplitArrivals];  // zero between launches
+static __device__ __align__(256) float split_scratch[kWorkspaces * kSplitScratchFloats];
+static __device__ unsigned split_arrivals[kWorkspaces * kSplitArrivals];  // zero between launches
 
 namespace tilemix {
 namespace {
@@ -1892,12 +1896,30 @@ bool split_pays(const AttnParams& p, bool precise, std::int64_t longest, std::in
     return saved_us > 1.05 * (4.5 + 0.75 * partial_mb);
 }
 
+struct Workspace {
+    hipEvent_t done = nullptr;
+    bool recorded = false;
+    hipStream_t stream = nullptr;  // of the last call
+    std::uint64_t used = 0;        // that call's number
+};
+
 struct SplitDevice {
     float* scratch = nullptr;
     unsigned* arrivals = nullptr;
-    hipEvent_t done = nullptr;
-    bool recorded = false;
+    Workspace workspaces[kWorkspaces];
+    std::uint64_t calls = 0;
 };
+
+// The stream's own workspace, else the least recently used one. (A handle may
+// name another stream than it did, so every call waits for the event.)
+int choose_workspace(const SplitDevice& device, hipStream_t stream) {
+    int oldest = 0;
+    for (int i = 0; i < kWorkspaces; ++i) {
+        if (device.workspaces[i].recorded && device.workspaces[i].stream == stream) return i;
+        if (device.workspaces[i].used < device.workspaces[oldest].used) oldest = i;
+    }
+    return oldest;
+}
 
 std::mutex& split_lock() {
     static std::mutex lock;
@@ -1952,15 +1974,17 @@ int workspace_device(hipStream_t stream) {
 }
 
 // Calls launch(scratch, arrivals), which enqueues kernels on `stream` that use
-// the workspace of `device` (the current one), ordered after the previous
-// call's and before the next one's.
+// one workspace of `device` (the current one), ordered after that workspace's
+// previous call and before its next one.
 template <typename Launch>
 hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
     std::lock_guard<std::mutex> guard(split_lock());
     SplitDevice& state = split_devices()[device];
     hipError_t status = hipSuccess;
-    if (!state.scratch || !state.arrivals || !state.done) {
-        // First split call on this device: another thread may be capturing a
+    const int chosen = choose_workspace(state, stream);
+    Workspace& workspace = state.workspaces[chosen];
+    if (!state.scratch || !state.arrivals || !workspace.done) {
+        // First split call on this device or workspace: another thread may be capturing a
         // graph in global mode, which would reject these runtime calls (they
         // enqueue no work), so this thread's capture mode is relaxed around
         // them and then restored.
@@ -1976,20 +2000,23 @@ hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
             status = hipGetSymbolAddress(&address, HIP_SYMBOL(split_arrivals));
             if (status == hipSuccess) state.arrivals = static_cast<unsigned*>(address);
         }
-        if (status == hipSuccess && !state.done) status = hipEventCreateWithFlags(&state.done, hipEventDisableTiming | hipEventDisableSystemFence);
+        if (status == hipSuccess && !workspace.done)
+            status = hipEventCreateWithFlags(&workspace.done, hipEventDisableTiming | hipEventDisableSystemFence);
         const hipError_t restored = hipThreadExchangeStreamCaptureMode(&mode);
         if (status != hipSuccess) return status;
         if (restored != hipSuccess) return restored;
     }
-    if (state.recorded) {
-        status = hipStreamWaitEvent(stream, state.done, 0);
+    if (workspace.recorded) {
+        status = hipStreamWaitEvent(stream, workspace.done, 0);
         if (status != hipSuccess) return status;
     }
-    status = launch(state.scratch, state.arrivals);
+    status = launch(state.scratch + chosen * kSplitScratchFloats, state.arrivals + chosen * kSplitArrivals);
     if (status != hipSuccess) return status;
-    status = hipEventRecord(state.done, stream);
+    status = hipEventRecord(workspace.done, stream);
     if (status != hipSuccess) return status;
-    state.recorded = true;
+    workspace.recorded = true;
+    workspace.stream = stream;
+    workspace.used = ++state.calls;
     return hipSuccess;
 }
 
