@@ -4,7 +4,8 @@ and without a causal mask, ranges past the diagonal, skipped cells and rows
 without a visible key, both P.V forms, every load width, output types and
 layouts, against the fp64 TileMix oracle (2e-3 / 2e-4 for the fast P.V,
 1e-5 + 1e-4|x| for the precise one), and the call with verification outputs
-against the one without, to the bit.
+against the one without, to the bit (Q8, K8 and the scales, cleared before each
+call, too).
 """
 from __future__ import annotations
 
@@ -55,6 +56,8 @@ def test_batched_split_vs_oracle(tm, oracle_lib, cuda, case):
     ks = torch.empty((heads, (N + 63) // 64), dtype=torch.int16, device="cuda:0")
     outs = []
     for traced in (False, True):
+        for t in (Q8, K8, qs, ks):
+            t.fill_(99)
         O = laid_out(torch.full((heads, M, d), 96.0, dtype=o_type, device="cuda:0"))
         trace = torch.full(codes.shape, 9, dtype=torch.uint8, device="cuda:0")
         args = tm.BatchedArgs(
@@ -69,12 +72,16 @@ def test_batched_split_vs_oracle(tm, oracle_lib, cuda, case):
         outs.append(O.float().cpu().numpy())
         if traced:
             assert np.array_equal(host(trace), codes)
+        for h in range(heads):
+            q8, q_s = oracle_lib.quantize(q[h], 128)
+            k8, k_s = oracle_lib.quantize(k[h], 64)
+            assert np.array_equal(host(Q8)[h], q8) and np.array_equal(host(K8)[h], k8)
+            assert np.array_equal(host(qs)[h].view(np.uint16), q_s)
+            assert np.array_equal(host(ks)[h].view(np.uint16), k_s)
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
     for h in range(heads):
         q8, q_s = oracle_lib.quantize(q[h], 128)
         k8, k_s = oracle_lib.quantize(k[h], 64)
-        assert np.array_equal(host(Q8)[h], q8) and np.array_equal(host(K8)[h], k8)
-        assert np.array_equal(host(qs)[h].view(np.uint16), q_s)
         want = oracle_lib.tilemix(q[h], k[h], v[h], q8, k8, q_s, k_s, codes[h], float(np.float32(d ** -0.5)), causal)
         got = outs[0][h]
         if precise:

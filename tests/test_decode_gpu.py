@@ -5,10 +5,12 @@ The shapes sit where that kernel can go wrong: the edges of a 32-key step, of a
 workgroup's range of steps and of the split over workgroups, every width of
 load that d and the alignment allow, one and sixteen rows, routes that change
 from cell to cell, skipped cells and heads with no visible key, each quantize
-mode, output type and layout. Every head is followed by NaN rows. Bounds are
-those of the batched sweep: 1e-5 + 1e-4|x| with precise P.V, max-abs 2e-3 and
-mean-abs 2e-4 with probabilities rounded to fp16 (plus half an ulp of a 16-bit
-O: 2^-9 |x| for bf16, 2^-12 |x| for fp16).
+mode, output type and layout; keys and values of more than 128 MiB, which are
+read with a non-temporal hint and by four or eight waves; NaN and infinity in Q.
+Every head is followed by NaN rows. Bounds are those of the batched sweep: 1e-5 +
+1e-4|x| with precise P.V, max-abs 2e-3 and mean-abs 2e-4 with probabilities
+rounded to fp16 (plus the rounding of a 16-bit O: at most 2^-8 |x| for bf16, 2^-11
+|x| for fp16).
 """
 from __future__ import annotations
 
@@ -213,3 +215,97 @@ def test_decode_under_graph_capture(tm, oracle_lib, cuda):
         tm.check(tm.attention_batched(args))  # eager, split, between the replays
         torch.cuda.synchronize()
         _check(oracle_lib, c, p, b)
+
+
+# heads, M, N, d, routed, precise, out: more than 128 MiB of keys and values. From the top: four waves with the
+# hint (64 steps a workgroup), eight with it (47), four at d <= 64, precise, 8-byte K8 rows, and rows in dword pieces.
+LARGE = [
+    (32, 4, 16384, 128, True, False, "f32"), (100, 4, 3000, 128, True, False, "bf16"), (64, 2, 9000, 64, True, False, "f32"),
+    (40, 3, 11000, 112, True, True, "f32"), (32, 16, 17000, 72, False, False, "f32"), (32, 2, 16500, 100, True, False, "f32"),
+    (256, 1, 1100, 128, False, True, "f32"), (520, 4, 700, 102, True, False, "f32"), (520, 4, 700, 128, True, False, "f32"),
+]
+
+
+@pytest.mark.parametrize("case", LARGE, ids=["-".join(map(str, c)) for c in LARGE])
+def test_decode_large(tm, oracle_lib, cuda, case):
+    import torch
+
+    from tilemix import routing
+
+    heads, M, N, d, routed, precise, out = case
+    assert heads * N * d * 4 > 128 << 20
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(heads + N)
+    Q, K, V = (torch.randn(heads, r, d, generator=gen, device="cuda", dtype=torch.float16) for r in (M, N, N))
+    O = torch.full((heads, M, d), 96.0, dtype=torch.bfloat16 if out == "bf16" else torch.float32, device="cuda")
+    codes = [_codes(np.random.default_rng(h), N, 2, 0.2, routed) for h in range(heads)]
+    options = dict(quantize=0)
+    if routed:
+        packed = [routing.pack_cells(x, 2) for x in codes]
+        empty = np.zeros(routing.word_count(M, N, 2), np.uint64)
+        K8 = torch.empty((heads, N, d), dtype=torch.int8, device="cuda")
+        ks = torch.empty((heads, (N + 63) // 64), dtype=torch.int16, device="cuda")
+        options = dict(quantize=1, route_words=dev(np.concatenate([r for r, _ in packed])),
+                       skip_words=dev(np.concatenate([empty if s is None else s for _, s in packed])), K8=K8,
+                       k_scales=ks)
+    print(f"large decode {case}", flush=True)
+    tm.check(tm.attention_batched(tm.BatchedArgs(
+        Q=Q, K=K, V=V, O=O, heads=heads, M=M, N=N, d=d, score_scale=d ** -0.5, precise=precise, key_tiles_per_group=2,
+        o_dtype=2 if out == "bf16" else 0, **options)))
+    torch.cuda.synchronize()
+    got = O.float().cpu().numpy().astype(np.float64)
+    assert np.isfinite(got).all()
+    for h in (0, heads // 2, heads - 1):
+        q, k, v = (host(x[h]) for x in (Q, K, V))
+        q8, q_s = oracle_lib.quantize(q, 128)
+        k8, k_s = oracle_lib.quantize(k, 64)
+        want = oracle_lib.tilemix(q, k, v, q8, k8, q_s, k_s, codes[h], float(np.float32(d ** -0.5)))
+        err = np.maximum(np.abs(got[h] - want) - (2.0 ** -8 * np.abs(want) if out == "bf16" else 0.0), 0.0)
+        if precise:
+            assert (err <= 1e-5 + 1e-4 * np.abs(want)).all(), (h, float(err.max()))
+        else:
+            assert err.max() <= 2e-3 and err.mean() <= 2e-4, (h, float(err.max()), float(err.mean()))
+
+
+@pytest.mark.parametrize("heads,M,N,d", [(3, 16, 700, 128), (2, 5, 3000, 64), (2, 9, 513, 72), (2, 16, 900, 100),
+                                         (3, 4, 1200, 33)])
+def test_decode_special_values_in_q(tm, oracle_lib, cuda, heads, M, N, d):
+    """Q quantized in the kernel, with a NaN in every head's block, the last of all NaN, the first also with the
+    largest fp16 value: Q8 and the scales are the quantizer's, and rows without a NaN are the oracle's."""
+    import torch
+
+    from tilemix import routing
+
+    rng = np.random.default_rng(N + d)
+    q, k, v = (oracle_lib.float_to_half(rng.standard_normal((heads, r, d)).astype(np.float32)) for r in (M, N, N))
+    for h in range(heads):
+        q[h, (3 * h + 1) % M, (7 * h) % d] = 0x7E00 if h % 2 else 0xFE00
+    q[0, 0, d - 1] = 0xFBFF
+    q[heads - 1] = 0x7E00
+    codes = [_codes(rng, N, 1, 0.0, True) for _ in range(heads)]
+    route = dev(np.concatenate([routing.pack_cells(x, 1)[0] for x in codes]))
+    Q, K, V = (dev_half(x) for x in (q, k, v))
+    outs = dict(Q8=torch.full((heads, M, d), 99, dtype=torch.int8, device="cuda"),
+                K8=torch.full((heads, N, d), 99, dtype=torch.int8, device="cuda"),
+                q_scales=torch.full((heads, 1), 99, dtype=torch.int16, device="cuda"),
+                k_scales=torch.full((heads, (N + 63) // 64), 99, dtype=torch.int16, device="cuda"))
+    wanted = {n: torch.empty_like(t) for n, t in outs.items()}
+    tm.check(tm.quantize_tilemix_qk_batched(Q, K, *wanted.values(), heads, M, N, d))
+    O = torch.full((heads, M, d), 96.0, device="cuda")
+    print(f"decode, NaN in Q: {heads} x {M} x {N} x {d}", flush=True)
+    tm.check(tm.attention_batched(tm.BatchedArgs(Q=Q, K=K, V=V, O=O, heads=heads, M=M, N=N, d=d, score_scale=d ** -0.5,
+                                                 precise=True, key_tiles_per_group=1, quantize=1, route_words=route,
+                                                 **outs)))
+    torch.cuda.synchronize()
+    for n in outs:
+        assert torch.equal(outs[n], wanted[n]), n
+    got = O.cpu().numpy()
+    for h in range(heads):
+        q8, q_s = oracle_lib.quantize(q[h], 128)
+        k8, k_s = oracle_lib.quantize(k[h], 64)
+        assert np.array_equal(host(outs["Q8"])[h], q8) and np.array_equal(host(outs["q_scales"])[h].view(np.uint16), q_s)
+        bad = ((q[h] & 0x7FFF) > 0x7C00).any(axis=1)
+        assert np.isnan(got[h][bad]).all() and np.isfinite(got[h][~bad]).all()
+        with np.errstate(invalid="ignore"):
+            want = oracle_lib.tilemix(q[h], k[h], v[h], q8, k8, q_s, k_s, codes[h], float(np.float32(d ** -0.5)))
+        assert (np.abs(got[h] - want)[~bad] <= (1e-5 + 1e-4 * np.abs(want))[~bad]).all()
