@@ -49,8 +49,8 @@ tilemix::AttnParams call(int heads, int M, int N, int d, bool causal) {
 
 // The 256-row kernel: never for heads of one 128-row block, never in more
 // rounds of workgroups than the 128-row kernel's, never for a causal walk of
-// fewer than 32 tiles however many keys there are; and the measured calls on
-// both sides of the line.
+// fewer than 32 tiles (64 at 64 features) however many keys there are; and the
+// measured calls on both sides of the line.
 void wide_kernel_rule() {
     using namespace tilemix;
     constexpr int kUnits = 256;
@@ -79,6 +79,19 @@ void wide_kernel_rule() {
     expect(48, 3000, 3000, 128, false, false);
     expect(64, 1024, 1024, 128, false, false);
     expect(16, 4096, 4096, 128, true, false);
+    expect(64, 4096, 4096, 64, true, true);
+    expect(128, 2048, 2048, 64, true, false);
+    expect(128, 2048, 2048, 128, true, true);
+    // A causal call with skipped tiles keeps the 128-row kernel up to 64 features.
+    const std::uint64_t words = 0;
+    for (int d : {40, 64, 112, 128}) {
+        AttnParams p = call(64, 4096, 4096, d, true);
+        p.skip_words = &words;
+        if (wide_pays(p, kUnits) != (d > 64)) {
+            std::printf("wide_pays(causal with skipped tiles, d %d) is not %d\n", d, d > 64);
+            ++failures;
+        }
+    }
 }
 
 // The decode kernel: up to one head per CU, and beyond that for rows of at most

@@ -26,7 +26,8 @@ CASES = {
     "d128": (32, 2048, 2048, 128, 2, False, 0.0, 4, "f32", "hsd", 1),
     "d64-cells-skip": (64, 1000, 2049, 64, 1, False, 0.3, 1, "f32", "hsd", 1),
     "causal-cells": (64, 2048, 2048, 128, 3, True, 0.1, 1, "f32", "hsd", 1),
-    "causal-d64-ragged": (64, 2047, 2047, 64, 2, True, 0.2, 4, "f32", "shd", 1),
+    "causal-d64-ragged": (64, 4095, 4095, 64, 2, True, 0.0, 4, "f32", "shd", 1),
+    "causal-d112-skip": (64, 2047, 2047, 112, 2, True, 0.2, 4, "f32", "shd", 1),
     "odd-blocks-d112": (128, 300, 2100, 112, 2, False, 0.3, 4, "f32", "hsd", 1),
     "windows-odd-count": (64, 1024, 4100, 128, 2, False, 0.0, 8, "bf16", "hsd", 1),
     "negative-scale": (32, 2048, 2300, 128, 2, False, 0.0, 4, "f16", "shd", -1),

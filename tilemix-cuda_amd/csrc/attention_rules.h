@@ -41,15 +41,18 @@ inline constexpr int kWideMaxTiles = 1024;  // key tiles that attention_wide_ker
 // One block a head: 512 x 128 187.4 | 225.4, 252 x 128 127 | 144, 256 x 128 125 |
 // 114, 256 x 64 x 2048 routed 59.8 | 71.8, 232 x 128 x 3000 x 64 59.0 | 63.1, 256
 // x 128 x 2048 x 64 39.5 | 35.7: no rule on sizes alone separates them. Causal
-// walks of 16 tiles, 256 x 1024 x 64 over 4096 keys: 65.7 | 73.0.
+// walks of 16 tiles, 256 x 1024 x 64 over 4096 keys: 65.7 | 73.0; of 32, 128 x
+// 2048 x 64 routed 111.3 | 114.7, x 128 173 | 167. Causal with skipped tiles
+// (three-way), which its waves wait for one another over: 64 x 4096 x 64 172.4 |
+// 176.8, 128 x 2048 x 64 102.8 | 110.6, x 128 157.6 | 157.9.
 inline bool wide_pays(const AttnParams& p, int compute_units) {
-    constexpr int kLongWalk = 32;  // key tiles
+    const int long_walk = p.causal && p.d <= 64 ? 64 : 32;  // key tiles
     const int tiles = (p.N - 1) / kTileKeys + 1;
     const int walk = p.causal ? std::min<std::int64_t>(tiles, std::int64_t{kRowsPerGroup / kTileKeys} * p.q_blocks) : tiles;
-    if (compute_units <= 0 || walk < kLongWalk || tiles > kWideMaxTiles) return false;
+    if (compute_units <= 0 || walk < long_walk || tiles > kWideMaxTiles) return false;
     if (p.q_blocks < 2 || (p.reverse_slots > 0 && p.q_blocks % 2 != 0)) return false;
     const std::int64_t workgroups = static_cast<std::int64_t>(p.heads) * ((p.q_blocks + 1) / 2);
-    if (p.causal) return workgroups >= 2 * static_cast<std::int64_t>(compute_units);
+    if (p.causal) return workgroups >= 2 * static_cast<std::int64_t>(compute_units) && !(p.skip_words && p.d <= 64);
     // Whole rounds: at most a tenth of the last one empty.
     const std::int64_t rounds = (workgroups + compute_units - 1) / compute_units;
     const std::int64_t slots = std::int64_t{kGroupsPerCU} * compute_units;
