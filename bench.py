@@ -220,7 +220,7 @@ def main() -> int:
         },
         "roofline": {
             "bound": "mfma",
-            "kernel": "attention_kernel",
+            "kernel": attention_kernel_name(w, args.precise),
             "achieved": round(achieved, 3),
             "peak": round(blended_peak, 3),
             "unit": "TFLOP/s",
@@ -428,8 +428,15 @@ def per_head_bench(args) -> dict:
                          "note": "time per round includes the quantizer launches"}}
 
 
+def attention_kernel_name(w, precise: bool) -> str:
+    """The kernel that the library's launch rules (csrc/attention_rules.h) choose for the workload:
+    the 128-row kernel for the tiny one and for precise P.V, else the 256-row kernel."""
+    return "attention_kernel" if precise or w.index == 1 else "attention_wide_kernel"
+
+
 # Sources whose change invalidates a recorded traffic measurement.
 STAMPED_SOURCES = ["tilemix-cuda_amd/csrc/attention.hip", "tilemix-cuda_amd/csrc/attention_common.h",
+                   "tilemix-cuda_amd/csrc/attention_rules.h",
                    "tilemix-cuda_amd/csrc/tilemix_device.h", "tilemix-cuda_amd/csrc/tilemix_launch.h",
                    "tilemix-cuda_amd/csrc/quantize.hip", "tilemix-cuda_amd/build.py"]
 
@@ -515,7 +522,7 @@ def measured_traffic(workload: str):
     path = ROOT / "profiles" / "traffic.json"
     if not path.exists():
         return None
-    entries = json.loads(path.read_text()).get("attention_kernel") or []
+    entries = json.loads(path.read_text()).get("attention") or []
     entry = next((e for e in entries if e.get("workload") == workload), None)
     if entry is None:
         return None

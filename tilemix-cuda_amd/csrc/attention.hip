@@ -1209,10 +1209,17 @@ __global__ __launch_bounds__(kThreadsPerGroup, kGroupsPerCU) void attention_kern
 // half of the kernel's time.)
 // What bounds it, at 128 features, dense (32 heads x 8192: 1033 us, 1.06
 // PFLOP/s; 1064 us with attention_kernel): about 1800 cycles a slot at 1.79 GHz
-// under the power limit. The matrix slot alone takes 1540 (1024 of them MFMAs;
-// the LDS reads of V's transposed fragments, at half the rate of K's, take
-// longer than the P.V MFMAs they feed), the vector slot alone 1500 (32
-// exponentials at 16 cycles, 110 other instructions). Interleaving P.V with the
+// under the power limit. Counted (GRBM_GUI_ACTIVE over the slots of a CU's
+// rounds): 1690 cycles a slot for 32 heads x 16384 with three quarters INT8, MFMA
+// busy 49 % of SIMD cycles; 1710 and 36 % for 32 x 8192 three-way; at 64 features
+// 1850, prologue and epilogue included, and 24 % (64 x 2048). The matrix slot
+// alone takes 1540 (1024 of them MFMAs; the LDS reads of V's transposed
+// fragments, at half the rate of K's, take longer than the P.V MFMAs they feed),
+// the vector slot alone 1500 (32 exponentials at 16 cycles, 110 other
+// instructions): from copies of the kernel with the other slot's work left out.
+// A slot ends in a barrier of all eight waves, so it takes as long as its slowest
+// wave: what a wave saves on an INT8 or skipped cell is lost there unless all
+// save it. Interleaving P.V with the
 // scores MFMA by MFMA spilled 160 registers at 128 features and was 3 % slower
 // at 64; three tile buffers of each were no faster.
 constexpr int kWideThreads = 512;

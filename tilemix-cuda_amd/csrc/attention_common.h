@@ -70,8 +70,10 @@ struct AttnParams {
     float score_scale;
     // Key-range split (splits > 1): workgroup b takes tiles [s * split_tiles,
     // (s + 1) * split_tiles) of item b / splits (s = b % splits) and writes
-    // its unnormalised O rows to part_o ([splits][M][d] fp32) and its row
-    // maximum and sum (log2 domain) to part_ml ([splits][M][2]) instead of O.
+    // its unnormalised O rows to part_o ([heads][splits][M][d] fp32) and its row
+    // maximum and sum (log2 domain) to part_ml ([heads][splits][M][2]) instead
+    // of O. Decode: tiles are its steps of 32 keys, and rows of part_o hold
+    // 64 * ceil(d / 64) floats. part_o null: the ranges in turn.
     int splits;
     int split_tiles;
     float* part_o;

@@ -33,7 +33,8 @@ inline constexpr int kWideMaxTiles = 1024;  // key tiles that attention_wide_ker
 // 32 x 2048 routed 53.3 | 51.1; 64 x 4096 causal 180.3 | 175.9; 16 x 2048 37.5 |
 // 39.6; 64 x 1024 25.8 | 26.2. 128 features: 32 x 16384 routed 3551 | 3363; 32 x
 // 8192 three-way 787 | 755; 32 x 8192 dense 1064 | 1033, causal 530 | 517; 64 x
-// 4096 causal 288.4 | 284.5; 16 x 4096 causal 106.3 | 108.2; 48 x 3000 (2.25
+// 4096 causal dense 288.4 | 284.5, routed in a band with the K quantizer 311.1 |
+// 310.8 on one box and 306.2 | 300.9 on another; 16 x 4096 causal 106.3 | 108.2; 48 x 3000 (2.25
 // rounds) 258.4 | 263.5; 64 x 1024 46.8 | 48.0; 16 x 2048 48.6 | 53.5. Precise
 // P.V, whose matrix slot is twice as long: 32 x 4096 causal 203.8 | 207.2.
 // Rows x 4096 keys x 128 features: 256 heads x 129 136.7 | 128.5; 256 x 300 247.8

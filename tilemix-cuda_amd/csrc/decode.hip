@@ -12,8 +12,11 @@
 //    (plan_decode) and, inside a workgroup, over its waves, 32 keys
 //    (one routing cell: M <= 16 rows are one cell tall) per wave and step;
 //  * a wave reads its keys and values straight into registers - no LDS, no
-//    barrier, the next step's 8 to 16 KiB in flight while one is computed, so
-//    up to 128 KiB per CU;
+//    barrier - and asks for the next step's 8 to 16 KiB before it computes one.
+//    As compiled, little of that stays in flight: above 64 features a part of
+//    the step's keys is kept in scratch memory (80 bytes a lane), and every
+//    variant waits for most of the loads just issued before the current step's
+//    MFMAs, so what hides the latency is the CU's other waves;
 //  * scores are S^T = K Q^T with v_mfma_f32_16x16x32_f16 or
 //    v_mfma_i32_16x16x64_i8 on 16 keys x 16 query rows. Lane (r, g) =
 //    (lane % 16, lane / 16) holds features 64 m + 16 g .. + 15 of key r as two
@@ -33,7 +36,8 @@
 // probabilities (precise: hi + lo), row sums of exactly those.
 //
 // Measured (MI355X, 32 heads x 4 rows x 16384 keys x 128, half the key tiles
-// INT8, 235 MB read): 428 us per call with the prefill kernel, 54 us here.
+// INT8, 235 MB read): 430 us per call with the prefill kernel, 54 to 55 us here
+// (4.3 TB/s; a large copy reaches 5.2).
 
 #include "attention_common.h"
 #include "tilemix_capi.h"
