@@ -128,3 +128,43 @@ def test_captured_split_call_equals_eager(tm, cuda, name):
         torch.cuda.synchronize()
         same(eager, captured, f"replay {replay}")
         same(eager, again, f"eager call after replay {replay}")
+
+
+@pytest.mark.parametrize("name", ["chunk-routed", "causal-d64-skip", "d100", "decode", "decode-d72"])
+def test_captured_verification_outputs(tm, cuda, name):
+    """The routing trace and the int32 dots of a captured split call, and O beside them."""
+    import torch
+
+    heads, M, N, d, causal, precise = CASES[name][:6]
+    Q, K, V, route, skip, laid_out = _problem(name)
+    Q8, K8 = (torch.empty((heads, rows, d), dtype=torch.int8, device="cuda") for rows in (M, N))
+    qs, ks = (torch.empty((heads, -(-rows // b)), dtype=torch.int16, device="cuda") for rows, b in ((M, 128), (N, 64)))
+    O = laid_out(torch.empty((heads, M, d), device="cuda"))
+    trace = torch.empty((heads, (M + 15) // 16, (N + 31) // 32), dtype=torch.uint8, device="cuda")
+    dots = torch.empty((heads, M, N), dtype=torch.int32, device="cuda")
+    args = tm.BatchedArgs(
+        Q=Q, K=K, V=V, O=O, heads=heads, M=M, N=N, d=d, score_scale=d ** -0.5, causal=causal, precise=precise, quantize=1,
+        route_words=route, skip_words=skip, key_tiles_per_group=2, Q8=Q8, K8=K8, q_scales=qs, k_scales=ks,
+        decoded_bits=trace, score_dots=dots, q_head_stride=Q.stride(0), k_head_stride=K.stride(0),
+        v_head_stride=V.stride(0), o_head_stride=O.stride(0), q_row_stride=Q.stride(1), k_row_stride=K.stride(1),
+        v_row_stride=V.stride(1), o_row_stride=O.stride(1))
+
+    def cleared():
+        for t in (O, trace, dots):
+            t.fill_(77)
+        torch.cuda.synchronize()
+
+    print(f"graph bits {name}: verification outputs", flush=True)
+    cleared()
+    tm.check(tm.attention_batched(args))
+    torch.cuda.synchronize()
+    eager = [t.clone() for t in (O, trace, dots)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tm.check(tm.attention_batched(args))
+    for replay in range(2):
+        cleared()
+        graph.replay()
+        torch.cuda.synchronize()
+        for what, a, b in zip(("O", "trace", "dots"), eager, (O, trace, dots)):
+            assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)), f"{what}, replay {replay}"
