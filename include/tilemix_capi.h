@@ -69,15 +69,16 @@ int tilemix_quantize_qk(const uint16_t* Q, const uint16_t* K, int8_t* Q8, int8_t
  * through its event (each waits for the previous one's merge): those of up to
  * four streams do not wait for one another, a further stream's wait for the
  * stream that used its array last. A call made while
- * `stream` is being captured into a graph uses neither array nor event: one
- * workgroup takes the ranges of a block in turn, and the replay equals the
- * eager call to the bit.
+ * `stream` is being captured into a graph uses neither array nor event and
+ * takes the unsplit launch.
  * tilemix_attention_batched splits a call of few, long row blocks (at least 16
- * key tiles) in the same way where that saves time.
+ * key tiles) in the same way where that saves time; under capture one workgroup
+ * takes the ranges of a block in turn, and the replay equals the eager call to
+ * the bit.
  * A call of M <= 16 query rows (here and in tilemix_attention_batched without
  * a causal mask) is served by a kernel of its own, which splits the keys of
  * its heads over workgroups of the same launch through the same workspace,
- * ordered, and under capture in turn, in the same way.
+ * ordered in the same way, and in turn, with the same bits, under capture.
  */
 int tilemix_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* V, float* O,
                       int M, int N, int d, float score_scale, void* stream,

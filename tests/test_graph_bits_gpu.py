@@ -4,9 +4,9 @@ keys in turn, so every replay equals the eager call to the bit, in every output.
 
 Batched splits (ragged, causal, routed with skipped cells, precise, every load
 width, 16-bit outputs, more ranges than one batch of the merge), split decode
-(four and eight waves, every load width, heads without a visible key) and the
-per-head call; the eager call runs again between the replays, and a repeated
-eager call gives the same bits too.
+(four and eight waves, every load width, heads without a visible key; the
+per-head call of 16 rows among them); the eager call runs again between the
+replays, and a repeated eager call gives the same bits too.
 """
 from __future__ import annotations
 
@@ -34,8 +34,8 @@ CASES = {
     "decode-d100": (2, 7, 3000, 100, False, True, 0.0, "f32", "hsd", False),
     "decode-d121": (2, 3, 2500, 121, False, False, None, "f32", "hsd", False),
     "decode-four-waves": (16, 4, 33000, 128, False, False, 0.0, "f32", "hsd", False),
-    "per-head": (1, 1000, 2500, 128, False, True, 0.0, "f32", "hsd", True),
-    "per-head-dense": (1, 777, 3001, 48, False, True, None, "f32", "hsd", True),
+    "per-head-decode": (1, 16, 2500, 128, False, True, 0.0, "f32", "hsd", True),
+    "precise-d48": (1, 777, 3001, 48, False, True, None, "f32", "hsd", False),
 }
 
 

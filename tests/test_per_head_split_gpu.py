@@ -9,8 +9,8 @@ library's fixed device workspace).
 * Ragged shapes and both O alignments (vector / element-wise combine) against
   the oracle, with the routing trace and INT32 dots exact; two of them have
   more splits than the combine takes in one batch (64 and 47).
-* A call made while its stream is captured into a graph uses no workspace and
-  no event (the ranges in turn): every replay equals the first, and the oracle.
+* A call made while its stream is captured into a graph takes the plain launch
+  (no workspace, no event): every replay equals the first, and the oracle.
 """
 from __future__ import annotations
 

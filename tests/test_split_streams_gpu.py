@@ -62,7 +62,7 @@ def test_a_held_stream_holds_up_no_other(tm, cuda):
     import torch
 
     calls = _calls(tm, 4)
-    ticks = _hold_ticks(0.5)
+    ticks = _hold_ticks(1.0)
     held, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(8)]
     done = [torch.cuda.Event() for _ in others]
     # Streams that share a hardware queue with the held one wait for it by themselves.
@@ -73,7 +73,7 @@ def test_a_held_stream_holds_up_no_other(tm, cuda):
         with torch.cuda.stream(stream):
             torch.zeros(1, device="cuda")
         event.record(stream)
-    beside = [s for s, free in zip(others, _finished(done, 0.3)) if free][:3]
+    beside = [s for s, free in zip(others, _finished(done, 0.5)) if free][:3]
     torch.cuda.synchronize()
     assert beside, "no stream runs beside the held one"
     print(f"split calls on {len(beside)} streams beside a held one", flush=True)
@@ -83,7 +83,7 @@ def test_a_held_stream_holds_up_no_other(tm, cuda):
     for stream, event, (call, _, _) in zip([held] + beside, done, calls):
         call(stream)
         event.record(stream)
-    finished = _finished(done[1:], 0.4)
+    finished = _finished(done[1:], 0.8)
     still_held = not done[0].query()
     torch.cuda.synchronize()
     assert all(finished) and still_held, (finished, still_held)

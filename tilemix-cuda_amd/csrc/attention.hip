@@ -1855,7 +1855,7 @@ hipError_t launch_attention(AttnParams p, int units, bool precise, hipStream_t s
 // concurrent streams never share a copy at once, and up to kWorkspaces of them
 // do not wait for one another (with one copy, a split call waited for all that
 // any stream had queued before its last one). Calls made while their stream is
-// being captured into a graph use none and take the same ranges of keys in turn.
+// being captured into a graph use none.
 static constexpr int kWorkspaces = 4;  // as many as hardware queues, HIP's default
 static constexpr std::size_t kSplitScratchFloats = std::size_t{8} << 20;  // 32 MiB each
 static constexpr std::size_t kSplitArrivals = 1024;
@@ -1877,13 +1877,18 @@ namespace {
 // 16.1 | 18.7, 19.8, -; 4 x 2048 causal x 128 46.5 | 26.1, 26.0, 28.2; 16 x
 // 128 x 4096 x 128 80.4 | 32.3, 28.7, 31.6; 8 x 512 x 8192 x 128 168.6 | 36.4,
 // 35.1, 35.0.
+// in_turn: a call without a workspace takes the ranges in turn, for the split
+// call's bits, which batched calls keep under capture; the per-head call, which
+// never promised them, takes the faster unsplit launch there (captured, 4096 x
+// 4096 x 128 116 us against 135, 1000 x 1003 x 128 37.7 against 46.7).
 struct SplitRule {
     int tiles;
     int longest;
     bool weigh;
+    bool in_turn;
 };
-constexpr SplitRule kSplitHead{2, 8, false};
-constexpr SplitRule kSplitBatch{4, 16, true};
+constexpr SplitRule kSplitHead{2, 8, false, false};
+constexpr SplitRule kSplitBatch{4, 16, true, true};
 
 // Whether a split saves more than it costs, from the calls measured above and
 // below. A lone workgroup of a CU walks a tile in about 0.5 + d / 160 us (half
@@ -2031,15 +2036,16 @@ hipError_t with_workspace(int device, hipStream_t stream, Launch&& launch) {
 // 128-row block when choose_split_tiles says so: the attention kernel writes
 // each split's partial rows to the workspace, split_combine_kernel merges them
 // into O, both on `stream`. Where the workspace is not to be used, one workgroup
-// takes a block's ranges in turn, to the same bits.
+// takes a block's ranges in turn, to the same bits, or all its keys at once
+// (SplitRule::in_turn).
 hipError_t launch_attention_split(AttnParams p, int units, bool precise, const SplitRule& rule, hipStream_t stream) {
     const int split_tiles = choose_split_tiles(p, precise, units, rule);
-    if (split_tiles == 0) return launch_attention(p, units, precise, stream);
+    const int device = split_tiles > 0 ? workspace_device(stream) : -1;
+    if (device < 0 && (split_tiles == 0 || !rule.in_turn)) return launch_attention(p, units, precise, stream);
     int tiles = (p.N - 1) / kTileKeys + 1;
     if (p.causal) tiles = std::min(tiles, p.q_blocks * (kRowsPerGroup / kTileKeys));
     p.split_tiles = split_tiles;
     p.splits = (tiles + split_tiles - 1) / split_tiles;
-    const int device = workspace_device(stream);
     if (device < 0) return launch_attention(p, units, precise, stream);  // the ranges in turn
     return with_workspace(device, stream, [&](float* scratch, unsigned*) {
         p.part_o = scratch;
